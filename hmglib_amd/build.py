@@ -14,7 +14,8 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libhmglib.so")
-SOURCES = ["prims.hip", "morton.hip", "tree.hip", "aca.hip", "schedule.hip", "mvp.hip", "mixed.hip",
+SOURCES = ["prims.hip", "morton.hip", "tree.hip", "aca.hip",
+           "aca_reg_exp.hip", "aca_reg_gauss.hip", "aca_reg_gauss_ref.hip", "schedule.hip", "mvp.hip", "mixed.hip",
            "api.hip", "server.hip", "store.hip", "batch.hip",
            "noalloc.hip", "mvp_multi.hip"]
 ARCH = os.environ.get("HMG_OFFLOAD_ARCH", "gfx950")

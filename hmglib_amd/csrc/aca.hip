@@ -1,5 +1,7 @@
-// aca.hip -- batched adaptive cross approximation, one wavefront per admissible
-// block, all rank steps inside one launch (no host round trips).
+// aca.hip -- batched adaptive cross approximation, one team of wavefronts per admissible
+// block, all rank steps inside one launch.  This file holds the rules, the launches and
+// the memory form (factors in their own storage, for the kernels, dimensions and ranks
+// that the register form of aca_reg.h does not take).
 //
 // Semantics follow the reference's batched ACA (linear_algebra.cu:3684-4012,
 // kernels :918-1147, :963-1018, :2009-2222) with the pivot race at :985 resolved
@@ -13,13 +15,13 @@
 // The 2-norm is a wavefront FP64 reduction; the argmax a (|v|, index, v) butterfly.
 #include <algorithm>
 
+#include "aca_reg.h"
 #include "hmg_internal.h"
 #include "kernel_eval.h"
 
 namespace hmg {
 
 namespace {
-
 
 __device__ __forceinline__ double wave_sum(double v)
 {
@@ -176,11 +178,7 @@ struct Team {
 // r % 5 == 0; mode 2: checked at every step.  Stop after rank step r when
 // ||u_r|| ||v_r|| <= c ||U V^T||_F over the first r+1 terms, c = eps (1-eta) /
 // (1+eps) (mode 1) or eps (mode 2).  ||U V^T||_F^2 is kept as a running sum:
-// + 2 sum_{l<r} (u_l.u_r)(v_l.v_r) + ||u_r||^2 ||v_r||^2.
-struct AcaTol {
-    int mode;
-    double c;
-};
+// + 2 sum_{l<r} (u_l.u_r)(v_l.v_r) + ||u_r||^2 ||v_r||^2.  (AcaTol, aca_reg.h)
 
 // Rows scanned at once when the residual-row search rejects a row, and the
 // largest rank step that scans (its U terms are staged per wavefront in LDS;
@@ -622,38 +620,35 @@ __device__ void aca_block(const Team<NW>& team, Coords c1, Coords c2, const Kern
 // wavefront keep sixteen rank terms' loads in flight (and the tolerance stop's
 // cross terms) without scratch memory.
 constexpr int kAcaTeam = 4;
-template <class T, int KIND, bool TOL>
+template <int KIND, bool TOL>
 __global__ void __launch_bounds__(kAcaTeam * kWave) __attribute__((amdgpu_waves_per_eu(3)))
-aca_kernel(Coords c1, Coords c2, KernelParams kp, const int4* __restrict__ blk,
-           const work_item* __restrict__ items, const int* __restrict__ list,
-           int nbig, int nsmall, const int* __restrict__ kb, const int64_t* __restrict__ uoff,
-           const int* __restrict__ ldu, const int64_t* __restrict__ voff, const int* __restrict__ ldv,
-           T* __restrict__ U, T* __restrict__ V, T* const* __restrict__ ublk, T* const* __restrict__ vblk,
-           int* __restrict__ keff, int tie_last, int scan, AcaTol tol)
+aca_kernel(AcaArgs g, int nbig, int nsmall)
 {
     __shared__ double s_v[kAcaTeam * kCrossCols];
     __shared__ int s_i[kAcaTeam];
     __shared__ double s_x[kAcaTeam];
-    __shared__ T sU[kAcaTeam][kScanRows * kScanL];
+    __shared__ double sU[kAcaTeam][kScanRows * kScanL];
     __shared__ double sX[kAcaTeam][kScanRows * MAX_POINT_DIMENSION];
     __shared__ double sBox[kAcaTeam][2 * MAX_POINT_DIMENSION];
     __shared__ double sVn[kAcaTeam][kScanL];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     // large blocks first: their long rank loops start at once
     if ((int)blockIdx.x < nbig) {
-        const int a = list[blockIdx.x];
+        const int a = g.list[blockIdx.x];
         const Team<kAcaTeam> team{s_v, s_i, s_x};
-        aca_block<T, kAcaTeam, KIND, TOL>(team, c1, c2, kp, blk[a], kb[a], ldv[a], ldu[a],
-                                          ublk ? ublk[a] : U + uoff[a], vblk ? vblk[a] : V + voff[a],
-                                     keff + a, tie_last, scan, sU[w], sX[w], sBox[w], sVn[w], items[a], tol);
+        aca_block<double, kAcaTeam, KIND, TOL>(team, g.c1, g.c2, g.kp, g.blk[a], g.kb[a], g.ldv[a], g.ldu[a],
+                                               g.ublk ? g.ublk[a] : g.U + g.uoff[a],
+                                               g.vblk ? g.vblk[a] : g.V + g.voff[a], g.keff + a, g.tie_last,
+                                               g.scan, sU[w], sX[w], sBox[w], sVn[w], g.items[a], g.tol);
     } else {
         const int q = ((int)blockIdx.x - nbig) * kAcaTeam + w;
         if (q >= nsmall) return;
-        const int a = list[nbig + q];
+        const int a = g.list[nbig + q];
         const Team<1> team{nullptr, nullptr, nullptr};
-        aca_block<T, 1, KIND, TOL>(team, c1, c2, kp, blk[a], kb[a], ldv[a], ldu[a],
-                                   ublk ? ublk[a] : U + uoff[a], vblk ? vblk[a] : V + voff[a],
-                              keff + a, tie_last, scan, sU[w], sX[w], sBox[w], sVn[w], items[a], tol);
+        aca_block<double, 1, KIND, TOL>(team, g.c1, g.c2, g.kp, g.blk[a], g.kb[a], g.ldv[a], g.ldu[a],
+                                        g.ublk ? g.ublk[a] : g.U + g.uoff[a], g.vblk ? g.vblk[a] : g.V + g.voff[a],
+                                        g.keff + a, g.tie_last, g.scan, sU[w], sX[w], sBox[w], sVn[w], g.items[a],
+                                        g.tol);
     }
 }
 
@@ -662,94 +657,332 @@ aca_kernel(Coords c1, Coords c2, KernelParams kp, const int4* __restrict__ blk,
 // (m1 x m2 x rank work when most rows are rejected) set the length of the build.
 // Two wavefronts per SIMD leave room for every value in registers (no scratch).
 constexpr int kAcaHuge = 8;
-template <class T, int KIND, bool TOL>
+template <int KIND, bool TOL>
 __global__ void __launch_bounds__(kAcaHuge * kWave) __attribute__((amdgpu_waves_per_eu(2)))
-aca_huge_kernel(Coords c1, Coords c2, KernelParams kp, const int4* __restrict__ blk,
-                const work_item* __restrict__ items, const int* __restrict__ list,
-                const int* __restrict__ kb, const int64_t* __restrict__ uoff, const int* __restrict__ ldu,
-                const int64_t* __restrict__ voff, const int* __restrict__ ldv, T* __restrict__ U,
-                T* __restrict__ V, T* const* __restrict__ ublk, T* const* __restrict__ vblk,
-                int* __restrict__ keff, int tie_last, int scan, AcaTol tol)
+aca_huge_kernel(AcaArgs g)
 {
     __shared__ double s_v[kAcaHuge * kCrossCols];
     __shared__ int s_i[kAcaHuge];
     __shared__ double s_x[kAcaHuge];
-    __shared__ T sU[kAcaHuge][2 * kScanRows * kScanL];
+    __shared__ double sU[kAcaHuge][2 * kScanRows * kScanL];
     __shared__ double sX[kAcaHuge][2 * kScanRows * MAX_POINT_DIMENSION];
     __shared__ double sBox[kAcaHuge][2 * MAX_POINT_DIMENSION];
     __shared__ double sVn[kAcaHuge][kScanL];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int a = list[blockIdx.x];
+    const int a = g.list[blockIdx.x];
     const Team<kAcaHuge> team{s_v, s_i, s_x};
-    aca_block<T, kAcaHuge, KIND, TOL>(team, c1, c2, kp, blk[a], kb[a], ldv[a], ldu[a],
-                                      ublk ? ublk[a] : U + uoff[a], vblk ? vblk[a] : V + voff[a],
-                                      keff + a, tie_last, scan, sU[w], sX[w], sBox[w], sVn[w], items[a], tol);
+    aca_block<double, kAcaHuge, KIND, TOL>(team, g.c1, g.c2, g.kp, g.blk[a], g.kb[a], g.ldv[a], g.ldu[a],
+                                           g.ublk ? g.ublk[a] : g.U + g.uoff[a],
+                                           g.vblk ? g.vblk[a] : g.V + g.voff[a], g.keff + a, g.tie_last, g.scan,
+                                           sU[w], sX[w], sBox[w], sVn[w], g.items[a], g.tol);
 }
 
 }  // namespace
 
-// Block class of the ACA launches: 0 = huge (an 8-wavefront workgroup, launched
-// beside the rest), 1 = large (a 4-wavefront workgroup), 2 = one wavefront.
-static int aca_class(const Engine& eng, int a)
+// Block classes of the ACA launches, in list order: 0 = huge (memory form, an
+// 8-wavefront workgroup), 1 = large (memory form, a 4-wavefront workgroup), 2 = one
+// wavefront (memory form); register form (aca_reg.h): 3, 4 = wide teams of 8 and 4
+// wavefronts, 5 .. = teams of kRegWaves.
+constexpr int kClasses = 14;
+constexpr int kRegClass = 3;
+constexpr int kWide = 2;  // wide classes
+// Team sizes.  Clusters of about 2^j points are the rule (halving a set of any size), so
+// there is a size at each power of two and one just above it.  16, 8 and 4 fill a compute
+// unit at four wavefronts per SIMD, 12 and 3 at three; 9 is alone on its compute unit
+// (times: aca_reg_kernel.h).
+constexpr int kRegWaves[kClasses - kRegClass] = {8, 4, 16, 12, 9, 8, 5, 4, 3, 2, 1};
+// Wide blocks of more rows plus columns run on 8 wavefronts (one workgroup per compute
+// unit: the few largest set the length of a build), smaller ones on 4 (three per compute
+// unit hide each other's waits).
+constexpr int64_t kWideEntries = 8192;
+// rounds after which the teams run the searches themselves (a block needs one round per
+// long search; the few blocks with many would otherwise each cost the rest a round trip)
+constexpr int kAcaRounds = 64;
+// Rejected rows in a row after which a block is suspended.  A team of the register form
+// tries a row in about a microsecond (four at a time) against some hundred for a round
+// trip; a wide one takes up to thirty per row, and the blocks suspended once mostly have
+// long searches again.
+constexpr int kRegTries = 64, kWideTries = 32, kWideRetries = 8;
+constexpr int kAcaBlind = 4;  // rounds between two looks at the queues
+// bound of a wide class' slabs together
+constexpr int64_t kSlabBytes = (int64_t)3 << 30;
+
+static int aca_class(const Engine& eng, const KernelParams& kp, int a)
 {
     const int4 b = eng.h_blk[eng.ndense + a];
-    const int64_t e = (int64_t)(b.y - b.x + 1) + (b.w - b.z + 1);
+    const int m1 = b.y - b.x + 1, m2 = b.w - b.z + 1;
+    const int64_t e = (int64_t)m1 + m2;
+    // The register form takes every block it has code for: ranks up to kRegRank, two or
+    // three dimensions, kernels whose evaluation leaves the factors their registers (the
+    // Bessel function does not).
+    if (eng.h_kb[a] <= kRegRank && (kp.dim == 2 || kp.dim == 3) && kp.kind != HMG_KERNEL_MATERN_REF) {
+        for (int c = kClasses - 1; c >= kRegClass + kWide; c--) {
+            if (std::max(m1, m2) <= kRegWaves[c - kRegClass] * kWave) return c;
+        }
+        return e > kWideEntries ? kRegClass : kRegClass + 1;
+    }
     return e > eng.aca_huge_entries ? 0 : e > eng.aca_big_entries ? 1 : 2;
 }
 
-// list[0 .. nhuge) huge blocks (their own launch on the second stream, joined
-// back), then nbig large and nsmall other blocks in one launch; factor offsets
-// uoff / voff (leading dims eng.ldu / eng.ldv) into U / V
-template <class T>
-static hmg_status aca_launch(Engine& eng, const Coords& c1, const Coords& c2, const KernelParams& kp,
-                             int tie_last, const int* list, int nhuge, int nbig, int nsmall, const int64_t* uoff,
-                             const int64_t* voff, T* U, T* V, int* keff, T* const* ublk = nullptr,
-                             T* const* vblk = nullptr)
+// blocks of one launch set per class, the largest rank and row count of each class, and
+// the slab elements of the wide ones
+struct AcaCounts {
+    int n[kClasses] = {0};
+    int kmax[kClasses] = {0};
+    int m1max[kClasses] = {0};
+    double work[kClasses] = {0.0};  // rows and columns times rank
+    int64_t slab[kWide] = {0};
+};
+
+// appends the blocks of `members` (ACA block indices) to list in class order (the wide
+// ones by decreasing size: they are taken from the list one by one)
+static AcaCounts aca_order(const Engine& eng, const KernelParams& kp, const std::vector<int>& members,
+                           int few, std::vector<int>& list)
 {
-    const int scan = eng.aca_row_scan ? 1 : 0;
-    const int4* blk = eng.blk.p + eng.ndense;
+    AcaCounts c;
+    std::vector<unsigned char> cls(members.size());
+    for (size_t q = 0; q < members.size(); q++) {
+        const int i = aca_class(eng, kp, members[q]);
+        cls[q] = (unsigned char)i;
+        c.n[i]++;
+        c.kmax[i] = std::max(c.kmax[i], eng.h_kb[members[q]]);
+    }
+    // teams of 8 and 4 whose ranks go past their on-chip terms, too few to fill the chip:
+    // with the 9 and 5 ones
+    // (build of 4096 points in 2D, k = 32: 2.1 ms so, 3.0 apart)
+    for (int i = kRegClass + kWide; i < kClasses; i++) {
+        const int w = kRegWaves[i - kRegClass];
+        if ((w != 8 && w != 4) || c.n[i] > few || c.kmax[i] <= 8 + kRegTail) continue;
+        for (auto& q : cls)
+            if (q == i) q--;
+        c.n[i - 1] += c.n[i];
+        c.kmax[i - 1] = std::max(c.kmax[i - 1], c.kmax[i]);
+        c.n[i] = 0;
+    }
+    for (size_t q = 0; q < members.size(); q++) {
+        const int a = members[q], i = cls[q];
+        const int4 b = eng.h_blk[eng.ndense + a];
+        c.work[i] += ((double)(b.y - b.x + 1) + (b.w - b.z + 1)) * eng.h_kb[a];
+        c.m1max[i] = std::max(c.m1max[i], b.y - b.x + 1);
+        if (i >= kRegClass && i < kRegClass + kWide)
+            c.slab[i - kRegClass] = std::max(c.slab[i - kRegClass], (int64_t)(b.w - b.z + 1) * eng.h_kb[a]);
+    }
+    size_t at[kClasses], run = list.size();
+    for (int i = 0; i < kClasses; i++) {
+        at[i] = run;
+        run += (size_t)c.n[i];
+    }
+    list.resize(run);
+    for (size_t q = 0; q < members.size(); q++) list[at[cls[q]]++] = members[q];
+    for (int i = kRegClass; i < kRegClass + kWide; i++)
+        std::stable_sort(list.begin() + (at[i] - c.n[i]), list.begin() + at[i], [&](int x, int y) {
+            const int4 p = eng.h_blk[eng.ndense + x], q = eng.h_blk[eng.ndense + y];
+            return (int64_t)(p.y - p.x) + (p.w - p.z) > (int64_t)(q.y - q.x) + (q.w - q.z);
+        });
+    return c;
+}
+
+static hmg_status reg_launch(const AcaArgs& g, int nw, bool wide, int kmax, hipStream_t s)
+{
+    switch (g.kp.kind) {
+    case HMG_KERNEL_GAUSSIAN:
+        return aca_reg_launch<HMG_KERNEL_GAUSSIAN>(g, nw, wide, kmax, s);
+    case HMG_KERNEL_GAUSSIAN_REF:
+        return aca_reg_launch<HMG_KERNEL_GAUSSIAN_REF>(g, nw, wide, kmax, s);
+    default:
+        return aca_reg_launch<HMG_KERNEL_EXPONENTIAL>(g, nw, wide, kmax, s);
+    }
+}
+
+static hmg_status search_launch(const AcaArgs& g, int maxm1, hipStream_t s)
+{
+    switch (g.kp.kind) {
+    case HMG_KERNEL_GAUSSIAN:
+        return aca_search_launch<HMG_KERNEL_GAUSSIAN>(g, maxm1, s);
+    case HMG_KERNEL_GAUSSIAN_REF:
+        return aca_search_launch<HMG_KERNEL_GAUSSIAN_REF>(g, maxm1, s);
+    default:
+        return aca_search_launch<HMG_KERNEL_EXPONENTIAL>(g, maxm1, s);
+    }
+}
+
+// Scratch of the register form's launches (grown as needed)
+struct AcaWork {
+    DevBuf<int> ints;  // [counters][two queues][row][found]
+    DevBuf<double> fro2, slabs[kWide];
+    int cus = 0;  // compute units
+    hmg_status init()
+    {
+        int dev = 0;
+        HMG_HIP(hipGetDevice(&dev));
+        HMG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        return HMG_OK;
+    }
+    // so many teams leave part of the chip idle (two per compute unit fill it)
+    int few() const { return 2 * cus; }
+};
+
+// The blocks of list[] (aca_order), factor offsets uoff / voff (leading dims eng.ldu /
+// eng.ldv) into U / V or block pointers ublk / vblk.  The classes are dealt to the
+// engine's two streams, the one with less work so far first, so that one's last workgroups
+// run beside the next; both are joined back.  Rounds: blocks that suspended themselves are searched and resumed until
+// none is left (each round raises the rank or the row of every one of them); the host
+// looks at the queues once per kAcaBlind rounds, the launches in between end at once
+// where their queue is empty.
+static hmg_status aca_launch(Engine& eng, const Coords& c1, const Coords& c2, const KernelParams& kp,
+                             int tie_last, const int* list, const AcaCounts& cnt, const int64_t* uoff,
+                             const int64_t* voff, double* U, double* V, int* keff, AcaWork& work,
+                             double* const* ublk = nullptr, double* const* vblk = nullptr)
+{
     const AcaTol tol{eng.aca_tol_mode, eng.aca_tol_c};
     hipStream_t s = eng.stream, s2 = eng.serialize ? eng.stream : eng.stream2;
-    const bool fork = nhuge > 0 && s2 != s;
-    if (nhuge > 0) {
-        if (fork) {
+    // counters of round q of a look: [q][class] blocks queued, [q][16 + wide class] work
+    constexpr int kRow = 32, kCounters = kRow * (kAcaBlind + 1);
+    int first[kClasses], nreg = 0, run = 0;
+    for (int c = 0; c < kClasses; c++) {
+        first[c] = run;
+        run += cnt.n[c];
+        if (c >= kRegClass) nreg += cnt.n[c];
+    }
+    int nslabs[kWide] = {0};
+    if (nreg > 0) {
+        const int na = eng.naca;
+        HMG_TRY(work.ints.alloc((size_t)kCounters + 2 * (size_t)nreg + 2 * (size_t)na));
+        HMG_TRY(work.fro2.alloc((size_t)na));
+        for (int i = 0; i < kWide; i++) {
+            if (cnt.n[kRegClass + i] == 0) continue;
+            const int64_t fit = std::max<int64_t>(kSlabBytes / (std::max<int64_t>(cnt.slab[i], 1) * 8), 1);
+            nslabs[i] = (int)std::min<int64_t>(std::min(cnt.n[kRegClass + i], std::max(work.cus, 1) * (i == 0 ? 1 : 3)),
+                                               fit);
+            // short of memory: fewer slabs; none at all: the memory form
+            while (nslabs[i] > 0 && work.slabs[i].alloc((size_t)(cnt.slab[i] * nslabs[i])) != HMG_OK) {
+                (void)hipGetLastError();
+                nslabs[i] /= 2;
+            }
+        }
+    }
+    int* const counters = work.ints.p;
+    AcaArgs g{};
+    g.c1 = c1;
+    g.c2 = c2;
+    g.kp = kp;
+    g.blk = eng.blk.p + eng.ndense;
+    g.items = eng.blocks.p + eng.ndense;
+    g.list = list;
+    g.kb = eng.kb.p;
+    g.uoff = uoff;
+    g.ldu = eng.ldu.p;
+    g.voff = voff;
+    g.ldv = eng.ldv.p;
+    g.U = U;
+    g.V = V;
+    g.ublk = ublk;
+    g.vblk = vblk;
+    g.keff = keff;
+    g.tie_last = tie_last;
+    g.scan = eng.aca_row_scan ? 1 : 0;
+    g.tol = tol;
+    g.few = work.few();
+    if (nreg > 0) {
+        g.row = counters + kCounters + 2 * (size_t)nreg;
+        g.found = g.row + eng.naca;
+        g.fro2 = work.fro2.p;
+        HMG_HIP(hipMemsetAsync(counters, 0, kCounters * sizeof(int), s));
+    }
+    const bool two = s2 != s;
+    auto fork = [&]() -> hmg_status {
+        if (two) {
             HMG_HIP(hipEventRecord(eng.ev_fork, s));
             HMG_HIP(hipStreamWaitEvent(s2, eng.ev_fork, 0));
         }
+        return HMG_OK;
+    };
+    auto join = [&]() -> hmg_status {
+        if (two) {
+            HMG_HIP(hipEventRecord(eng.ev_join, s2));
+            HMG_HIP(hipStreamWaitEvent(s, eng.ev_join, 0));
+        }
+        return HMG_OK;
+    };
+    HMG_TRY(fork());
+    if (cnt.n[0] > 0) {
         if (tol.mode != 0) {
-            HMG_DISPATCH_KIND(kp.kind, aca_huge_kernel<T, KIND, true><<<nhuge, kAcaHuge * kWave, 0, s2>>>(
-                                           c1, c2, kp, blk, eng.blocks.p + eng.ndense, list, eng.kb.p, uoff,
-                                           eng.ldu.p, voff, eng.ldv.p, U, V, ublk, vblk, keff, tie_last,
-                                           scan, tol));
+            HMG_DISPATCH_KIND(kp.kind, aca_huge_kernel<KIND, true><<<cnt.n[0], kAcaHuge * kWave, 0, s2>>>(g));
         } else {
-            HMG_DISPATCH_KIND(kp.kind, aca_huge_kernel<T, KIND, false><<<nhuge, kAcaHuge * kWave, 0, s2>>>(
-                                           c1, c2, kp, blk, eng.blocks.p + eng.ndense, list, eng.kb.p, uoff,
-                                           eng.ldu.p, voff, eng.ldv.p, U, V, ublk, vblk, keff, tie_last,
-                                           scan, tol));
+            HMG_DISPATCH_KIND(kp.kind, aca_huge_kernel<KIND, false><<<cnt.n[0], kAcaHuge * kWave, 0, s2>>>(g));
         }
         HMG_HIP(hipGetLastError());
-        if (fork) HMG_HIP(hipEventRecord(eng.ev_join, s2));
-        list += nhuge;
     }
+    const int nbig = cnt.n[1], nsmall = cnt.n[2];
     const unsigned grid = (unsigned)(nbig + (nsmall + kAcaTeam - 1) / kAcaTeam);
-    if (grid == 0) {
-        if (fork) HMG_HIP(hipStreamWaitEvent(s, eng.ev_join, 0));
-        return HMG_OK;
+    if (grid > 0) {
+        g.list = list + first[1];
+        if (tol.mode != 0) {
+            HMG_DISPATCH_KIND(kp.kind, aca_kernel<KIND, true><<<grid, kAcaTeam * kWave, eng.aca_lds_pad, s>>>(
+                                           g, nbig, nsmall));
+        } else {
+            HMG_DISPATCH_KIND(kp.kind, aca_kernel<KIND, false><<<grid, kAcaTeam * kWave, eng.aca_lds_pad, s>>>(
+                                           g, nbig, nsmall));
+        }
+        HMG_HIP(hipGetLastError());
     }
-    if (tol.mode != 0) {
-        HMG_DISPATCH_KIND(kp.kind, aca_kernel<T, KIND, true><<<grid, kAcaTeam * kWave, eng.aca_lds_pad, s>>>(
-                                       c1, c2, kp, blk, eng.blocks.p + eng.ndense, list, nbig, nsmall,
-                                       eng.kb.p, uoff, eng.ldu.p, voff, eng.ldv.p, U, V, ublk, vblk, keff, tie_last, scan,
-                                       tol));
-    } else {
-        HMG_DISPATCH_KIND(kp.kind, aca_kernel<T, KIND, false><<<grid, kAcaTeam * kWave, eng.aca_lds_pad, s>>>(
-                                       c1, c2, kp, blk, eng.blocks.p + eng.ndense, list, nbig, nsmall,
-                                       eng.kb.p, uoff, eng.ldu.p, voff, eng.ldv.p, U, V, ublk, vblk, keff, tie_last, scan,
-                                       tol));
+    int n[kClasses];
+    for (int c = 0; c < kClasses; c++) {
+        n[c] = cnt.n[c];
+        if (c < kRegClass || c >= kRegClass + kWide || n[c] == 0 || nslabs[c - kRegClass] > 0) continue;
+        g.list = list + first[c];
+        if (tol.mode != 0) {
+            HMG_DISPATCH_KIND(kp.kind, aca_huge_kernel<KIND, true><<<n[c], kAcaHuge * kWave, 0, s2>>>(g));
+        } else {
+            HMG_DISPATCH_KIND(kp.kind, aca_huge_kernel<KIND, false><<<n[c], kAcaHuge * kWave, 0, s2>>>(g));
+        }
+        HMG_HIP(hipGetLastError());
+        n[c] = 0;
     }
-    HMG_HIP(hipGetLastError());
-    if (fork) HMG_HIP(hipStreamWaitEvent(s, eng.ev_join, 0));
-    return HMG_OK;
+    for (int round = 0; nreg > 0;) {
+        // one look: the blocks themselves, or kAcaBlind rounds of the suspended ones
+        const int rounds = round == 0 ? 1 : kAcaBlind;
+        double load[2] = {0.0, 0.0};
+        for (int c = kRegClass; c < kClasses; c++) {
+            if (n[c] == 0) continue;
+            const bool wide = c < kRegClass + kWide;
+            const int to = load[0] <= load[1] ? 0 : 1;
+            load[to] += cnt.work[c] * n[c] / cnt.n[c];
+            hipStream_t sc = to == 0 ? s : s2;
+            const int at = first[c] - first[kRegClass];
+            for (int q = 0; q < rounds; q++) {
+                const int parity = (round + q) & 1;
+                g.list = round == 0 ? list + first[c] : counters + kCounters + (size_t)parity * nreg + at;
+                g.queue = counters + kCounters + (size_t)(1 - parity) * nreg + at;
+                g.nlist = n[c];
+                g.count = counters + q * kRow + c;
+                g.queued = counters + (q + 1) * kRow + c;
+                g.next = counters + q * kRow + 16 + (c - kRegClass);
+                g.resume = round > 0 ? 1 : 0;
+                g.suspend = g.scan && round < kAcaRounds ? 1 : 0;
+                g.tries = !wide ? kRegTries : round == 0 ? kWideTries : kWideRetries;
+                if (wide) {
+                    g.slabs = work.slabs[c - kRegClass].p;
+                    g.slab = cnt.slab[c - kRegClass];
+                    g.nslabs = nslabs[c - kRegClass];
+                }
+                if (round > 0) HMG_TRY(search_launch(g, cnt.m1max[c], sc));
+                HMG_TRY(reg_launch(g, kRegWaves[c - kRegClass], wide, cnt.kmax[c], sc));
+            }
+        }
+        round += rounds;
+        HMG_TRY(join());
+        if (!g.scan) return HMG_OK;
+        // the blocks queued by the look's last round are the first row of the next one
+        HMG_TRY(download_bytes(n, counters + rounds * kRow, sizeof(int) * kClasses, s));
+        bool any = false;
+        for (int c = kRegClass; c < kClasses; c++) any = any || n[c] > 0;
+        if (!any) return HMG_OK;
+        HMG_HIP(hipMemsetAsync(counters, 0, kCounters * sizeof(int), s));
+        HMG_TRY(upload_bytes(counters, n, sizeof(int) * kClasses, s));
+        HMG_TRY(fork());
+    }
+    return join();
 }
 
 hmg_status aca_build(Engine& eng, const Coords& c1, const Coords& c2, const KernelParams& kp, int k,
@@ -759,22 +992,17 @@ hmg_status aca_build(Engine& eng, const Coords& c1, const Coords& c2, const Kern
     const int na = eng.naca;
     if (na == 0) return HMG_OK;
     hipStream_t s = eng.stream;
-    // huge blocks, then large blocks (a workgroup each), then the rest (a wavefront each)
-    std::vector<int>& order = eng.h_aca_list;
-    order.clear();
-    order.reserve(na);
-    int cnt[3] = {0, 0, 0};
-    for (int cls = 0; cls < 3; cls++) {
-        const int before = (int)order.size();
-        for (int a = 0; a < na; a++)
-            if (aca_class(eng, a) == cls) order.push_back(a);
-        cnt[cls] = (int)order.size() - before;
-    }
+    std::vector<int> all(na);
+    for (int a = 0; a < na; a++) all[a] = a;
+    eng.h_aca_list.clear();
+    AcaWork work;
+    HMG_TRY(work.init());
+    const AcaCounts cnt = aca_order(eng, kp, all, work.few(), eng.h_aca_list);
     HMG_TRY(eng.aca_list.alloc(na));
-    HMG_TRY(upload_bytes(eng.aca_list.p, order.data(), sizeof(int) * na, s));
+    HMG_TRY(upload_bytes(eng.aca_list.p, eng.h_aca_list.data(), sizeof(int) * na, s));
     eng.prof.begin(PROF_ACA, s);
-    HMG_TRY(aca_launch<double>(eng, c1, c2, kp, tie_last, eng.aca_list.p, cnt[0], cnt[1], cnt[2], eng.uoff.p,
-                               eng.voff.p, U, V, keff, ublk, vblk));
+    HMG_TRY(aca_launch(eng, c1, c2, kp, tie_last, eng.aca_list.p, cnt, eng.uoff.p, eng.voff.p, U, V, keff, work,
+                       ublk, vblk));
     eng.prof.end(PROF_ACA, s);
     return HMG_OK;
 }
@@ -908,19 +1136,16 @@ hmg_status aca_build_mixed(Engine& eng, const Coords& c1, const Coords& c2, cons
     HMG_TRY(upload(d_svoff, svoff, s));
     HMG_TRY(upload(eng.ldu, ldu, s));
     HMG_TRY(upload(eng.ldv, ldv, s));
-    // per batch: its huge, then large blocks, then the rest (the ACA launches' order)
+    // per batch: its blocks in the ACA launches' class order
     std::vector<int> list;
     list.reserve(na);
-    std::vector<int> bptr(nb + 1, 0), bhuge(nb, 0), bbig(nb, 0);
+    std::vector<int> bptr(nb + 1, 0);
+    AcaWork work;
+    HMG_TRY(work.init());
+    std::vector<AcaCounts> cnt(nb);
     for (int q = 0; q < nb; q++) {
         bptr[q] = (int)list.size();
-        for (int cls = 0; cls < 3; cls++) {
-            const int before = (int)list.size();
-            for (const int a : members[q])
-                if (aca_class(eng, a) == cls) list.push_back(a);
-            if (cls == 0) bhuge[q] = (int)list.size() - before;
-            if (cls == 1) bbig[q] = (int)list.size() - before;
-        }
+        cnt[q] = aca_order(eng, kp, members[q], work.few(), list);
     }
     bptr[nb] = (int)list.size();
     HMG_TRY(upload(d_list, list, s));
@@ -928,8 +1153,8 @@ hmg_status aca_build_mixed(Engine& eng, const Coords& c1, const Coords& c2, cons
     for (int q = 0; q < nb; q++) {
         const int n = bptr[q + 1] - bptr[q];
         if (n == 0) continue;
-        HMG_TRY(aca_launch<double>(eng, c1, c2, kp, tie_last, d_list.p + bptr[q], bhuge[q], bbig[q],
-                                   n - bhuge[q] - bbig[q], d_suoff.p, d_svoff.p, S.p, S.p, eng.keff.p));
+        HMG_TRY(aca_launch(eng, c1, c2, kp, tie_last, d_list.p + bptr[q], cnt[q], d_suoff.p, d_svoff.p, S.p, S.p,
+                           eng.keff.p, work));
         mx_panel_kernel<<<n, kConvThreads, 0, s>>>(d_list.p + bptr[q], eng.blk.p + eng.ndense, eng.kb.p,
                                                   eng.keff.p, d_suoff.p, d_svoff.p, eng.mxp.p, S.p, Up, Vp);
         HMG_HIP(hipGetLastError());

@@ -226,18 +226,20 @@ hmg_status hmg_get_schedule(const struct h_matrix_data* data, int64_t out[11]);
  *   mode data->U and data->V point at the BF16 factor panels and a stored FP64
  *   near field is not used.
  * HMG_OPT_ACA_ROW_SCAN [1]: when the residual-row search of the ACA rejects a
- *   row, compute the norms of the following rows four at a time (rank steps up
- *   to 64) instead of one at a time, and give rank 0 without evaluating it to a
- *   block whose entries are provably all too small for any row to pass the
- *   search (decreasing kernels, bound from the points' bounding boxes).  The
+ *   row, leave a long search of a block to one over all such blocks together (a
+ *   lane per row) instead of one row after the other, and give rank 0 without
+ *   evaluating it to a block whose entries are provably all too small for any row
+ *   to pass the search (decreasing kernels, bound from the points' bounding boxes).  The
  *   factors are bitwise the same.
- * HMG_OPT_ACA_BIG_BLOCK [512]: admissible blocks with more rows plus columns
- *   than this run their ACA on a workgroup of 4 wavefronts instead of one
+ * HMG_OPT_ACA_BIG_BLOCK [512]: of the admissible blocks whose ACA keeps its
+ *   factors in memory (Matern kernels, ranks above 64, more than three
+ *   dimensions; the others take a team by their size), those with more rows plus
+ *   columns than this run their ACA on a workgroup of 4 wavefronts instead of one
  *   wavefront (row norms summed in another order; same factors up to the
  *   rounding of those norms).
- * HMG_OPT_ACA_HUGE_BLOCK [16384]: blocks with more rows plus columns than this
- *   run on a workgroup of 8 wavefronts, in a launch on the engine's second
- *   stream beside the others (same factors up to the rounding of the norms).
+ * HMG_OPT_ACA_HUGE_BLOCK [16384]: of the same blocks, those with more rows plus
+ *   columns than this run on a workgroup of 8 wavefronts, in a launch on the
+ *   engine's second stream beside the others (same factors up to the rounding of the norms).
  * HMG_OPT_ACA_TOLERANCE [0]: stopping rule of the ACA.  0: fixed rank k (the
  *   reference's batched path, whose epsilon is unused).  1: the reference's
  *   tolerance criterion (linear_algebra.cu:498-528 with the V'*V of :379
@@ -274,8 +276,8 @@ hmg_status hmg_get_schedule(const struct h_matrix_data* data, int64_t out[11]);
  * HMG_OPT_MIXED_ACA_PARTS [16]: mixed precision: the FP64 ACA runs in batches whose
  *   FP64 factors (before the split into BF16 panels) fill at most 1/parts of the
  *   factors' size (at least 1 GiB); results unchanged.
- * HMG_OPT_ACA_LDS_BYTES [0]: unused LDS each workgroup of the main ACA launch
- *   reserves, capping the blocks in flight per compute unit (their factor columns,
+ * HMG_OPT_ACA_LDS_BYTES [0]: unused LDS each workgroup of the main launch of the
+ *   same blocks reserves, capping the blocks in flight per compute unit (their factor columns,
  *   re-read at every rank step, then stay in cache); results unchanged. */
 #define HMG_OPT_NEAR_SYMMETRIC 1
 #define HMG_OPT_NEAR_LDS_BYTES 2

@@ -43,46 +43,48 @@ __device__ __forceinline__ double kernel_of_r2_k(const KernelParams& kp, double 
 
 // e^x for x <= 0 (the argument of the product kernels' entries), within 1 ulp:
 // Cody-Waite reduction x = n ln2 + r with ln2 split into two doubles (its double
-// and the double of the remainder), |r| <= ln2/2, the degree-13 Taylor polynomial
-// of e^r (truncation below 5e-18 relative) by Horner's rule, scaled by 2^n.
-// Arguments below -800 give 0 (e^-800 is below the smallest double).
+// and the double of the remainder), |r| <= ln2/2, then a polynomial of degree 12
+// by Horner's rule, scaled by 2^n.  n is read off the low word of x log2(e) + 1.5 2^52.
+// The polynomial is 1 + r + r^2/2 + r^3 q(r), q the interpolant of the remainder in the
+// ten Chebyshev nodes of the interval (10^-18 relative; the Taylor polynomial needs one
+// degree more for 4 10^-18).  Arguments below -800 give 0 (e^-800 is below the
+// smallest double).
 __device__ __forceinline__ double exp_nonpos(double x)
 {
     x = fmax(x, -800.0);
-    const double n = rint(x * 1.4426950408889634);
+    const double m = __fma_rn(x, 1.4426950408889634, 6755399441055744.0);
+    const double n = m - 6755399441055744.0;
     double r = __fma_rn(n, -0.6931471805599453, x);
     r = __fma_rn(n, -2.3190468138462996e-17, r);
-    double p = 1.6059043836821613e-10;  // 1/13!
-    p = __fma_rn(p, r, 2.08767569878681e-09);
-    p = __fma_rn(p, r, 2.505210838544172e-08);
-    p = __fma_rn(p, r, 2.755731922398589e-07);
-    p = __fma_rn(p, r, 2.7557319223985893e-06);
-    p = __fma_rn(p, r, 2.48015873015873e-05);
-    p = __fma_rn(p, r, 0.0001984126984126984);
-    p = __fma_rn(p, r, 0.001388888888888889);
-    p = __fma_rn(p, r, 0.008333333333333333);
+    double p = 2.0911229798760165e-09;
+    p = __fma_rn(p, r, 2.5100375929185925e-08);
+    p = __fma_rn(p, r, 2.755728298391084e-07);
+    p = __fma_rn(p, r, 2.7557268480106926e-06);
+    p = __fma_rn(p, r, 2.480158731713526e-05);
+    p = __fma_rn(p, r, 0.00019841269863040675);
+    p = __fma_rn(p, r, 0.0013888888888886554);
+    p = __fma_rn(p, r, 0.008333333333330065);
     p = __fma_rn(p, r, 0.041666666666666664);
-    p = __fma_rn(p, r, 0.16666666666666666);
+    p = __fma_rn(p, r, 0.16666666666666669);
     p = __fma_rn(p, r, 0.5);
     p = __fma_rn(p, r, 1.0);
     p = __fma_rn(p, r, 1.0);
-    return ldexp(p, (int)n);
+    return ldexp(p, __double2loint(m));
 }
 
-// sqrt(x) for finite x >= 0: the hardware reciprocal square root refined by a
-// Goldschmidt step and two Newton corrections of the root (g += (x - g^2) h)
+// sqrt(x) for finite x >= 0: the hardware reciprocal square root (22 bits; its infinity
+// at 0 made finite), a Goldschmidt step (44 bits) and one Newton correction of the root,
+// g += (x - g^2) h, whose error is its final rounding.  Correctly rounded in 5 10^6
+// random arguments, as with a refined h and a second correction.
 __device__ __forceinline__ double sqrt_nonneg(double x)
 {
-    const double y = __builtin_amdgcn_rsq(x);
-    double g = x * y, h = 0.5 * y;
+    const double y = fmin(__builtin_amdgcn_rsq(x), 1.0e300);
+    double g = x * y;
+    const double h = 0.5 * y;
     const double r = __fma_rn(-g, h, 0.5);
     g = __fma_rn(g, r, g);
-    h = __fma_rn(h, r, h);
-    double d = __fma_rn(-g, g, x);
-    g = __fma_rn(d, h, g);
-    d = __fma_rn(-g, g, x);
-    g = __fma_rn(d, h, g);
-    return x == 0.0 ? 0.0 : g;
+    const double d = __fma_rn(-g, g, x);
+    return __fma_rn(d, h, g);
 }
 
 // The entries of the FP64 products (near field, dense rows, stored near field):

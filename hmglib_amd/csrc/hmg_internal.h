@@ -441,10 +441,9 @@ struct Engine {
     // tuning: LDS bytes reserved per near-field workgroup (caps its occupancy so
     // the low-rank streams keep wave slots on every CU); run the near field on
     // the main stream instead (no overlap)
-    // 64 KB + the kernel's own 12 KB leave room for 2 near-field workgroups per CU
-    // (measured on MI355X at N = 2^20, 3D, symmetric near field: 42.8 ms per
-    // product vs 46.2 ms with 3 workgroups per CU and 57.9 ms without overlap)
-    int near_lds_pad = 64 * 1024;
+    // -1: the kernel's own choice (mvp.hip, mixed.hip)
+    int near_lds_pad = -1;
+    int near_pad(int own) const { return near_lds_pad >= 0 ? near_lds_pad : own; }
     bool serialize = false;
     // ACA: scan rejected rows of the residual-row search several at a time;
     // blocks with more rows plus columns than aca_big_entries get a workgroup

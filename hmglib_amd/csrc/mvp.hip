@@ -142,13 +142,21 @@ __device__ __forceinline__ double kernel_value(const KernelParams& kp, double r2
 // rows per lane) against the columns of its dense blocks, which are staged 64 at a
 // time through this wave's LDS slice.  NR rows per lane give NR independent
 // evaluation chains per staged column.  DIM = 0 means "dim at run time".
+// Bound by the FP64 issue rate: 41 slots an entry, 5.0 ms for 3.2 10^9 entries (of 8 10^11 a
+// second at the clock that such a stream of FMAs keeps).
 constexpr int kNearRows = 2 * kWave;
+// LDS reserved per near-field workgroup, which leaves wavefront slots to the low-rank
+// kernels beside it.  The matrix-free form needs its own (24 KB, six workgroups per compute
+// unit): 3D, N = 262144 7.7 ms with none, 8.1 with 32 KB, 10.0 with 64.  The stored one
+// streams: N = 50021 2.03 with none, 1.97 with 32, 2.11 with 64.
+constexpr int kFlyPad = 0, kStoredPad = 32 * 1024;
 
 // lane i receives lane (i + 1) mod 64 of v (DPP wave_rol:1)
 __device__ __forceinline__ double lane_rotate_down(double v)
 {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x134, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x134, 0xf, 0xf, false);
+    const int l = __double2loint(v), h = __double2hiint(v);
+    const int lo = __builtin_amdgcn_update_dpp(l, l, 0x134, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(h, h, 0x134, 0xf, 0xf, false);
     return __hiloint2double(hi, lo);
 }
 
@@ -171,7 +179,7 @@ template <int KIND, int DIM, bool REG, int NR>
 __device__ __forceinline__ void near_fly_item(const Coords& c1, const Coords& c2, const KernelParams& kp,
                                               const NearItem& it, const NearRef* __restrict__ refs,
                                               const double* __restrict__ xs,
-                                              double (*sh)[kWave], int lane, double* __restrict__ out,
+                                              double (*sh)[2 * kWave], int lane, double* __restrict__ out,
                                               double* __restrict__ P)
 {
     constexpr int kS = MAX_POINT_DIMENSION + 1;
@@ -189,7 +197,8 @@ __device__ __forceinline__ void near_fly_item(const Coords& c1, const Coords& c2
         for (int d = 0; d < MAX_POINT_DIMENSION; d++) xi[r][d] = d < dim ? c1.x[d][row[r]] : 0.0;
     }
     // symmetric refs: one column stream over all their columns, 64 columns staged
-    // at a time (lane L stages column L).  Step s pairs lane L with staged column
+    // at a time (lane L stages column L, twice, so that a step's column is at an offset
+    // known at compile time).  Step s pairs lane L with staged column
     // (L + s) mod 64; the column sums travel one lane down per step, so after 64
     // steps lane L holds the sum of column L over this item's rows.
     if (it.ncols_sym > 0) {
@@ -221,12 +230,13 @@ __device__ __forceinline__ void near_fly_item(const Coords& c1, const Coords& c2
             wave_barrier();
 #pragma unroll
             for (int d = 0; d < MAX_POINT_DIMENSION; d++)
-                if (d < dim) sh[d][lane] = c2.x[d][jj];
-            sh[kS - 1][lane] = j >= 0 ? xs[jj] : 0.0;
+                if (d < dim) sh[d][lane] = sh[d][lane + kWave] = c2.x[d][jj];
+            sh[kS - 1][lane] = sh[kS - 1][lane + kWave] = j >= 0 ? xs[jj] : 0.0;
             wave_barrier();
             double colacc = 0.0;
+#pragma unroll 2
             for (int s = 0; s < kWave; s++) {
-                const int c = (lane + s) & (kWave - 1);
+                const int c = lane + s;
                 double xj[MAX_POINT_DIMENSION];
 #pragma unroll
                 for (int d = 0; d < MAX_POINT_DIMENSION; d++) xj[d] = d < dim ? sh[d][c] : 0.0;
@@ -290,7 +300,7 @@ near_fly_kernel(Coords c1, Coords c2, KernelParams kp, const NearItem* __restric
                 const NearRef* __restrict__ refs, const double* __restrict__ xs,
                 double* __restrict__ Pnear, double* __restrict__ P)
 {
-    __shared__ double sh[kWaves][MAX_POINT_DIMENSION + 1][kWave];
+    __shared__ double sh[kWaves][MAX_POINT_DIMENSION + 1][2 * kWave];
     const int lane = threadIdx.x & (kWave - 1);
     const int w = wave_id();
     const int q = blockIdx.x * kWaves + w;
@@ -468,10 +478,10 @@ void launch_near_fly(bool reg, unsigned grid, hipStream_t s, const Coords& c1, c
 {
     double* Pnear = P + (int64_t)eng.n_lr_items * kTileRows;
     if (reg)
-        near_fly_kernel<KIND, DIM, true><<<grid, kThreads, eng.near_lds_pad, s>>>(
+        near_fly_kernel<KIND, DIM, true><<<grid, kThreads, eng.near_pad(kFlyPad), s>>>(
             c1, c2, kp, eng.fly_items.p, eng.n_fly_items, eng.fly_refs.p, xs, Pnear, P);
     else
-        near_fly_kernel<KIND, DIM, false><<<grid, kThreads, eng.near_lds_pad, s>>>(
+        near_fly_kernel<KIND, DIM, false><<<grid, kThreads, eng.near_pad(kFlyPad), s>>>(
             c1, c2, kp, eng.fly_items.p, eng.n_fly_items, eng.fly_refs.p, xs, Pnear, P);
 }
 
@@ -532,7 +542,7 @@ hmg_status hmvp_with(Engine& eng, const Coords& c1, const Coords& c2, const Kern
             const unsigned g = grid_for(n_items, kWaves);
             eng.prof.begin(PROF_NEAR, s2);
             if (dense_stored) {
-                near_stored_kernel<<<g, kThreads, eng.near_lds_pad, s2>>>(
+                near_stored_kernel<<<g, kThreads, eng.near_pad(kStoredPad), s2>>>(
                     eng.near_items.p, eng.n_near_items, eng.near_blk.p, eng.blk.p, eng.aoff.p, eng.A.p,
                     b.xs, b.P + (int64_t)eng.n_lr_items * kTileRows);
             } else {

@@ -28,7 +28,14 @@ namespace {
 
 constexpr int kSlice = kTileRows;          // rows per low-rank work item (one wavefront)
 constexpr int kNearSlice = 2 * kTileRows;  // rows per near-field work item (two per lane)
-constexpr int kNearChunkCols = 4096;       // near-field columns per work item
+// Near-field columns per work item (whole blocks): as many as give kNearItems items, between
+// these bounds.  An item is a wavefront's work and the chip holds 5000 to 8000 of them, so
+// with fewer items the last ones run on a nearly empty chip: 3D, N = 262144, matrix-free
+// 8.5 ms with 10^4 items of up to 3000 columns, 7.7 with 3.3 10^4 of 770, 8.6 with 10^5;
+// N = 65537 with 17 right-hand sides 10.3, 9.6, 9.9; stored N = 50021 2.9 ms with 4096
+// columns, 2.0 with 256.
+constexpr int kNearChunkMin = 256, kNearChunkMax = 4096;
+constexpr int64_t kNearItems = 32768;
 constexpr int kVChunkRows = 1024;          // points per V^T x work item (FP64)
 constexpr int kMxVChunkRows = 4096;        // points per V^T x work item (mixed precision)
 constexpr int kMxRows = kMxNearRows;       // rows per mixed-precision near-field item
@@ -79,13 +86,13 @@ void group_by_row(const std::vector<int4>& bl, int b0, int b1, int base, std::ve
     for (int b = b0; b < b1; b++) idx[fill[g_of[b - b0]]++] = b - base;
 }
 
-// cut a run of column counts into chunks of at most kNearChunkCols columns
-std::vector<int> column_chunks(const std::vector<int>& m2s)
+// cut a run of column counts into chunks of at most `chunk` columns
+std::vector<int> column_chunks(const std::vector<int>& m2s, int chunk)
 {
     std::vector<int> cut{0};
     int cols = 0;
     for (int q = 0; q < (int)m2s.size(); q++) {
-        if (cols > 0 && cols + m2s[q] > kNearChunkCols) {
+        if (cols > 0 && cols + m2s[q] > chunk) {
             cut.push_back(q);
             cols = 0;
         }
@@ -207,6 +214,13 @@ void build_mixed_near(Engine& eng)
     eng.n_mx_items = (int)eng.h_mx_items.size();
 }
 
+// chunk for row slices that see that many columns altogether
+int near_chunk(int64_t slice_cols)
+{
+    const int64_t c = round_up(std::max<int64_t>(slice_cols / kNearItems, 1), 64);
+    return (int)std::min<int64_t>(std::max<int64_t>(c, kNearChunkMin), kNearChunkMax);
+}
+
 }  // namespace
 
 hmg_status build_groups(Engine& eng)
@@ -219,6 +233,12 @@ hmg_status build_groups(Engine& eng)
     // stored near field: (dense row cluster, 128-row slice, chunk of its blocks)
     std::vector<int4>& items = eng.h_near_items;
     items.clear();
+    int64_t slice_cols = 0;
+    for (int b = 0; b < eng.ndense; b++) {
+        const int4 bl = eng.h_blk[b];
+        slice_cols += ((int64_t)(bl.y - bl.x) / kNearSlice + 1) * (bl.w - bl.z + 1);
+    }
+    const int chunk = near_chunk(slice_cols);
     for (int g = 0; g < ng; g++) {
         const int gb0 = eng.h_dgrp_ptr[g], gb1 = eng.h_dgrp_ptr[g + 1];
         const int4 first = eng.h_blk[eng.h_dgrp_blk[gb0]];
@@ -228,7 +248,7 @@ hmg_status build_groups(Engine& eng)
             const int4 b = eng.h_blk[eng.h_dgrp_blk[q]];
             m2s.push_back(b.w - b.z + 1);
         }
-        const std::vector<int> cut = column_chunks(m2s);
+        const std::vector<int> cut = column_chunks(m2s, chunk);
         for (int r0 = 0; r0 < m1; r0 += kNearSlice)
             for (size_t c = 0; c + 1 < cut.size(); c++)
                 items.push_back(make_int4(l1 + r0, std::min(kNearSlice, m1 - r0), gb0 + cut[c], gb0 + cut[c + 1]));
@@ -258,6 +278,8 @@ hmg_status build_groups(Engine& eng)
         if (!dense_set.count(PairKey{range_key(b.z, b.w), range_key(b.x, b.y)})) return 0;
         return b.x < b.z ? 1 : 2;
     };
+    // (a symmetric block stands for two)
+    const int fly_chunk = near_chunk(eng.near_sym ? slice_cols / 2 : slice_cols);
     std::vector<std::pair<int, int>> sym_refs;  // (fly ref index, dense block) awaiting a column slot
     for (int g = 0; g < ng; g++) {
         const int gb0 = eng.h_dgrp_ptr[g], gb1 = eng.h_dgrp_ptr[g + 1];
@@ -275,7 +297,7 @@ hmg_status build_groups(Engine& eng)
         if (order.empty()) continue;
         std::vector<int> m2s;
         for (int b : order) m2s.push_back(eng.h_blk[b].w - eng.h_blk[b].z + 1);
-        const std::vector<int> cut = column_chunks(m2s);
+        const std::vector<int> cut = column_chunks(m2s, fly_chunk);
         const int nplain = (int)plain.size();
         for (int r0 = 0; r0 < m1; r0 += kNearSlice) {
             for (size_t c = 0; c + 1 < cut.size(); c++) {

@@ -411,6 +411,10 @@ struct Engine {
     DevBuf<int4> near_items;                    // stored near field: {row0, nrows, b0, b1}
     DevBuf<int> near_blk;
     std::vector<int4> h_near_items;
+    // matrix-free near field: dense blocks per row cluster (those with row sums only, then
+    // from h_fly_sym on the symmetric ones); chunk size of the work items (0: none yet)
+    std::vector<int> h_fly_ptr, h_fly_sym, h_fly_blk;
+    int near_scale = 0;
     // matrix-free near field (symmetric when both sets are the same points)
     bool same_sets = false;                     // sorted coordinates bitwise equal
     bool near_sym_enabled = true;               // option: allow the symmetric form
@@ -675,6 +679,10 @@ struct MvpSizes {
     int64_t xs, Tp, T, P;
 };
 MvpSizes mvp_sizes(const Engine& eng);
+// the product without allocation: doubles of its fixed scratch (32 MiB; a product whose
+// buffers need more is refused), and those a product needs there
+constexpr int64_t kNoallocDoubles = (int64_t)1 << 22;
+int64_t noalloc_need(const MvpSizes& z);
 // hmvp with caller-provided buffers (allocates nothing)
 hmg_status hmvp_with(Engine& eng, const Coords& c1, const Coords& c2, const KernelParams& kp,
                      const uint64_t* order1, const uint64_t* order2, const double* x, double* y, int nrhs,

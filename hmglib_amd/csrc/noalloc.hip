@@ -4,7 +4,7 @@
 // computes for an H-matrix whose FP64 factors are precomputed, with the same
 // kernels, but its per-call buffers (x in sorted order, the V^T x partials, t,
 // and the partial sums every row adds up) live in a fixed device array of
-// kScratchDoubles doubles that the code object holds, instead of in memory the
+// kNoallocDoubles doubles that the code object holds, instead of in memory the
 // engine allocates on first use.  It calls no hipMalloc / hipFree and no
 // allocating library routine, so it is usable where allocation is not: under
 // stream capture, in serving loops that forbid it.
@@ -20,9 +20,7 @@
 namespace hmg {
 namespace {
 
-// 32 MiB: a product whose buffers need more is refused
-constexpr int64_t kScratchDoubles = (int64_t)1 << 22;
-__device__ __align__(256) double scratch[kScratchDoubles];
+__device__ __align__(256) double scratch[kNoallocDoubles];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -61,6 +59,9 @@ __global__ void fill_zero_kernel(double* __restrict__ p, int64_t n)
 inline int64_t aligned(int64_t n) { return (n + 31) / 32 * 32; }
 
 }  // namespace
+
+int64_t noalloc_need(const MvpSizes& z) { return aligned(z.xs) + aligned(z.Tp) + aligned(z.T) + aligned(z.P); }
+
 }  // namespace hmg
 
 using namespace hmg;
@@ -82,10 +83,10 @@ extern "C" hmg_status hmg_apply_h_matrix_mvp_noalloc(const double* X, double* Y,
     KernelParams kp;
     HMG_TRY(read_kernel(data, &kp));
     const MvpSizes z = mvp_sizes(*e);
-    const int64_t need = aligned(z.xs) + aligned(z.Tp) + aligned(z.T) + aligned(z.P);
-    if (need > kScratchDoubles) {
+    const int64_t need = noalloc_need(z);
+    if (need > kNoallocDoubles) {
         set_error("no-alloc product: this H-matrix needs " + std::to_string(need) +
-                  " doubles of per-call buffers; the fixed scratch holds " + std::to_string(kScratchDoubles));
+                  " doubles of per-call buffers; the fixed scratch holds " + std::to_string(kNoallocDoubles));
         return HMG_ERR_INVALID;
     }
     double* base;

@@ -230,33 +230,6 @@ hmg_status build_groups(Engine& eng)
     group_by_row(eng.h_blk, eng.ndense, eng.nblocks, eng.ndense, eng.h_cgrp_ptr, eng.h_cgrp_blk, true);
     const int ng = (int)eng.h_dgrp_ptr.size() - 1;
 
-    // stored near field: (dense row cluster, 128-row slice, chunk of its blocks)
-    std::vector<int4>& items = eng.h_near_items;
-    items.clear();
-    int64_t slice_cols = 0;
-    for (int b = 0; b < eng.ndense; b++) {
-        const int4 bl = eng.h_blk[b];
-        slice_cols += ((int64_t)(bl.y - bl.x) / kNearSlice + 1) * (bl.w - bl.z + 1);
-    }
-    const int chunk = near_chunk(slice_cols);
-    for (int g = 0; g < ng; g++) {
-        const int gb0 = eng.h_dgrp_ptr[g], gb1 = eng.h_dgrp_ptr[g + 1];
-        const int4 first = eng.h_blk[eng.h_dgrp_blk[gb0]];
-        const int l1 = first.x, m1 = first.y - first.x + 1;
-        std::vector<int> m2s;
-        for (int q = gb0; q < gb1; q++) {
-            const int4 b = eng.h_blk[eng.h_dgrp_blk[q]];
-            m2s.push_back(b.w - b.z + 1);
-        }
-        const std::vector<int> cut = column_chunks(m2s, chunk);
-        for (int r0 = 0; r0 < m1; r0 += kNearSlice)
-            for (size_t c = 0; c + 1 < cut.size(); c++)
-                items.push_back(make_int4(l1 + r0, std::min(kNearSlice, m1 - r0), gb0 + cut[c], gb0 + cut[c + 1]));
-    }
-    eng.n_near_items = (int)items.size();
-    HMG_TRY(upload(eng.near_items, items, eng.stream));
-    HMG_TRY(upload(eng.near_blk, eng.h_dgrp_blk, eng.stream));
-
     // matrix-free near field: transposed pairs when both sides are the same points
     std::unordered_set<PairKey, PairHash> dense_set;
     eng.near_sym = eng.same_sets && eng.near_sym_enabled;
@@ -267,9 +240,6 @@ hmg_status build_groups(Engine& eng)
             dense_set.insert(PairKey{range_key(bl.x, bl.y), range_key(bl.z, bl.w)});
         }
     }
-    eng.h_fly_items.clear();
-    eng.h_fly_refs.clear();
-    eng.near_evals = 0;
     // kind: 0 = row sums only, 1 = symmetric (row + column sums), 2 = covered by its transpose
     auto kind_of = [&](const int4& b) {
         if (!eng.near_sym) return 0;
@@ -278,27 +248,105 @@ hmg_status build_groups(Engine& eng)
         if (!dense_set.count(PairKey{range_key(b.z, b.w), range_key(b.x, b.y)})) return 0;
         return b.x < b.z ? 1 : 2;
     };
+    eng.h_fly_ptr.assign(1, 0);
+    eng.h_fly_sym.clear();
+    eng.h_fly_blk.clear();
+    for (int g = 0; g < ng; g++) {
+        std::vector<int> sym;
+        for (int q = eng.h_dgrp_ptr[g]; q < eng.h_dgrp_ptr[g + 1]; q++) {
+            const int b = eng.h_dgrp_blk[q];
+            const int k = kind_of(eng.h_blk[b]);
+            if (k == 0) eng.h_fly_blk.push_back(b);
+            else if (k == 1) sym.push_back(b);
+        }
+        eng.h_fly_sym.push_back((int)eng.h_fly_blk.size());
+        eng.h_fly_blk.insert(eng.h_fly_blk.end(), sym.begin(), sym.end());
+        eng.h_fly_ptr.push_back((int)eng.h_fly_blk.size());
+    }
+    eng.near_scale = 0;  // no work items yet (aca_layout)
+    return HMG_OK;
+}
+
+namespace {
+
+// column chunks of the near-field work items: the stored form's and the matrix-free
+// one's, at `scale` times their own size
+struct NearChunks {
+    int stored, fly;
+};
+NearChunks near_chunks(const Engine& eng, int scale)
+{
+    int64_t slice_cols = 0;
+    for (int b = 0; b < eng.ndense; b++) {
+        const int4 bl = eng.h_blk[b];
+        slice_cols += ((int64_t)(bl.y - bl.x) / kNearSlice + 1) * (bl.w - bl.z + 1);
+    }
     // (a symmetric block stands for two)
-    const int fly_chunk = near_chunk(eng.near_sym ? slice_cols / 2 : slice_cols);
-    std::vector<std::pair<int, int>> sym_refs;  // (fly ref index, dense block) awaiting a column slot
+    return NearChunks{std::min(near_chunk(slice_cols) * scale, kNearChunkMax),
+                      std::min(near_chunk(eng.near_sym ? slice_cols / 2 : slice_cols) * scale, kNearChunkMax)};
+}
+
+// columns of the blocks at [q0, q1) of a list
+std::vector<int> block_cols(const Engine& eng, const std::vector<int>& blk, int q0, int q1)
+{
+    std::vector<int> m2s;
+    m2s.reserve((size_t)(q1 - q0));
+    for (int q = q0; q < q1; q++) {
+        const int4 b = eng.h_blk[blk[q]];
+        m2s.push_back(b.w - b.z + 1);
+    }
+    return m2s;
+}
+
+// near-field work items at that scale: the larger of the two forms' numbers
+int64_t count_near(const Engine& eng, int scale)
+{
+    const NearChunks ch = near_chunks(eng, scale);
+    int64_t stored = 0, fly = 0;
+    for (int g = 0; g + 1 < (int)eng.h_dgrp_ptr.size(); g++) {
+        const int4 first = eng.h_blk[eng.h_dgrp_blk[eng.h_dgrp_ptr[g]]];
+        const int64_t slices = (first.y - first.x) / kNearSlice + 1;
+        auto cuts = [&](const std::vector<int>& blk, int q0, int q1, int chunk) -> int64_t {
+            return q0 == q1 ? 0 : (int64_t)column_chunks(block_cols(eng, blk, q0, q1), chunk).size() - 1;
+        };
+        stored += slices * cuts(eng.h_dgrp_blk, eng.h_dgrp_ptr[g], eng.h_dgrp_ptr[g + 1], ch.stored);
+        fly += slices * cuts(eng.h_fly_blk, eng.h_fly_ptr[g], eng.h_fly_ptr[g + 1], ch.fly);
+    }
+    return std::max(stored, fly);
+}
+
+// the near-field work items of both FP64 forms
+hmg_status split_near(Engine& eng, int scale)
+{
+    const NearChunks ch = near_chunks(eng, scale);
+    const int ng = (int)eng.h_dgrp_ptr.size() - 1;
+    // stored near field: (dense row cluster, 128-row slice, chunk of its blocks)
+    std::vector<int4>& items = eng.h_near_items;
+    items.clear();
     for (int g = 0; g < ng; g++) {
         const int gb0 = eng.h_dgrp_ptr[g], gb1 = eng.h_dgrp_ptr[g + 1];
         const int4 first = eng.h_blk[eng.h_dgrp_blk[gb0]];
         const int l1 = first.x, m1 = first.y - first.x + 1;
-        std::vector<int> plain, sym;
-        for (int q = gb0; q < gb1; q++) {
-            const int b = eng.h_dgrp_blk[q];
-            const int k = kind_of(eng.h_blk[b]);
-            if (k == 0) plain.push_back(b);
-            else if (k == 1) sym.push_back(b);
-        }
-        std::vector<int> order(plain);
-        order.insert(order.end(), sym.begin(), sym.end());
-        if (order.empty()) continue;
-        std::vector<int> m2s;
-        for (int b : order) m2s.push_back(eng.h_blk[b].w - eng.h_blk[b].z + 1);
-        const std::vector<int> cut = column_chunks(m2s, fly_chunk);
-        const int nplain = (int)plain.size();
+        const std::vector<int> cut = column_chunks(block_cols(eng, eng.h_dgrp_blk, gb0, gb1), ch.stored);
+        for (int r0 = 0; r0 < m1; r0 += kNearSlice)
+            for (size_t c = 0; c + 1 < cut.size(); c++)
+                items.push_back(make_int4(l1 + r0, std::min(kNearSlice, m1 - r0), gb0 + cut[c], gb0 + cut[c + 1]));
+    }
+    eng.n_near_items = (int)items.size();
+    HMG_TRY(upload(eng.near_items, items, eng.stream));
+    HMG_TRY(upload(eng.near_blk, eng.h_dgrp_blk, eng.stream));
+
+    eng.h_fly_items.clear();
+    eng.h_fly_refs.clear();
+    eng.near_evals = 0;
+    std::vector<std::pair<int, int>> sym_refs;  // (fly ref index, dense block) awaiting a column slot
+    for (int g = 0; g < ng; g++) {
+        const int gb0 = eng.h_fly_ptr[g], gb1 = eng.h_fly_ptr[g + 1], sym0 = eng.h_fly_sym[g];
+        if (gb0 == gb1) continue;
+        const int4 first = eng.h_blk[eng.h_dgrp_blk[eng.h_dgrp_ptr[g]]];
+        const int l1 = first.x, m1 = first.y - first.x + 1;
+        const std::vector<int> m2s = block_cols(eng, eng.h_fly_blk, gb0, gb1);
+        const std::vector<int> cut = column_chunks(m2s, ch.fly);
         for (int r0 = 0; r0 < m1; r0 += kNearSlice) {
             for (size_t c = 0; c + 1 < cut.size(); c++) {
                 NearItem it;
@@ -307,19 +355,21 @@ hmg_status build_groups(Engine& eng)
                 it.ref0 = (int)eng.h_fly_refs.size();
                 it.ref_sym = -1;
                 it.ncols_sym = 0;
+                int cols = 0;
                 for (int q = cut[c]; q < cut[c + 1]; q++) {
-                    if (q >= nplain && it.ref_sym < 0) it.ref_sym = (int)eng.h_fly_refs.size();
-                    const int4 b = eng.h_blk[order[q]];
-                    if (q >= nplain) {
-                        it.ncols_sym += b.w - b.z + 1;
-                        sym_refs.emplace_back((int)eng.h_fly_refs.size(), order[q]);
+                    const bool sym = gb0 + q >= sym0;
+                    if (sym && it.ref_sym < 0) it.ref_sym = (int)eng.h_fly_refs.size();
+                    const int blk = eng.h_fly_blk[gb0 + q];
+                    const int4 b = eng.h_blk[blk];
+                    if (sym) {
+                        it.ncols_sym += m2s[q];
+                        sym_refs.emplace_back((int)eng.h_fly_refs.size(), blk);
                     }
-                    eng.h_fly_refs.push_back(NearRef{b.z, b.w - b.z + 1, -1});
+                    eng.h_fly_refs.push_back(NearRef{b.z, m2s[q], -1});
+                    cols += m2s[q];
                 }
                 it.ref1 = (int)eng.h_fly_refs.size();
                 if (it.ref_sym < 0) it.ref_sym = it.ref1;
-                int cols = 0;
-                for (int q = cut[c]; q < cut[c + 1]; q++) cols += m2s[q];
                 eng.near_evals += (int64_t)it.nrows * cols;
                 eng.h_fly_items.push_back(it);
             }
@@ -344,9 +394,11 @@ hmg_status build_groups(Engine& eng)
         run += (int64_t)m2 * (int64_t)kv.second.size();
     }
     eng.n_col_slots = run;
-    HMG_HIP(hipStreamSynchronize(eng.stream));
+    eng.near_scale = scale;
     return HMG_OK;
 }
+
+}  // namespace
 
 hmg_status aca_layout(Engine& eng, int k, int prec)
 {
@@ -617,6 +669,23 @@ hmg_status aca_layout(Engine& eng, int k, int prec)
     // per slot (allocated by the product)
     const int64_t near0 = (int64_t)eng.n_lr_items * lrows;
     hipStream_t s = eng.stream;
+    // Short items need more partial sums, and the product without allocation has a fixed
+    // scratch for them: where the longest items fit there, they grow until they do (the
+    // column slots do not depend on them).
+    int scale = std::max(eng.near_scale, 1);
+    if (!mixed) {
+        if (eng.near_scale == 0) HMG_TRY(split_near(eng, 1));
+        auto fits = [&](int64_t nnear) {
+            MvpSizes z = mvp_sizes(eng);
+            z.P = std::max<int64_t>(near0 + nnear * kNearSlice + eng.n_col_slots, 1);
+            return noalloc_need(z) <= kNoallocDoubles;
+        };
+        scale = 1;
+        const int64_t own = eng.near_scale == 1 ? std::max(eng.n_near_items, eng.n_fly_items) : count_near(eng, 1);
+        if (!fits(own) && fits(count_near(eng, kNearChunkMax)))
+            for (scale = 2; !fits(count_near(eng, scale)); scale *= 2) {}
+    }
+    if (eng.near_scale != scale) HMG_TRY(split_near(eng, scale));
     const int n1 = eng.n[0];
     int64_t col0 = 0;
     if (!mixed) {

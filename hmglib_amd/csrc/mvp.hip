@@ -391,7 +391,8 @@ dense_fill_kernel(Coords c1, Coords c2, KernelParams kp, const int4* __restrict_
 // entries, as the near field is; a lane per row over all columns left the chip with two
 // wavefronts per compute unit.  N = 32768: 3D exponential 15.9 -> 1.21 ms (8.9 10^11 entries
 // a second), 2D Gaussian 0.85 ms.  Partial sums go to P[chunk * ld + row].
-// The short entries (kernel_of_r2_prod) are for finite squared distances; a block of
+// Squared distances round as dist2's, so that an entry stays within 2 ulps of one computed
+// from it.  The short entries (kernel_of_r2_prod) are for finite squared distances; a block of
 // columns or a row tile with a coordinate of 10^100 or more, or not a number, takes the
 // general ones, as do the reference kernels and, with a regularization, the blocks on the
 // diagonal.
@@ -449,8 +450,17 @@ full_kernel(Coords c1, Coords c2, KernelParams kp, const double* __restrict__ xs
                 for (int d = 0; d < MAX_POINT_DIMENSION; d++) xj[d] = d < dim ? sh[d][jj] : 0.0;
                 const double xv = sh[kS - 1][jj];
 #pragma unroll
-                for (int r = 0; r < 2; r++)
-                    acc[r] = __fma_rn(entry_value<KIND, DIM>(kp, xi[r], xj), xv, acc[r]);
+                for (int r = 0; r < 2; r++) {
+                    double r2 = 0.0;
+#pragma unroll
+                    for (int d = 0; d < MAX_POINT_DIMENSION; d++) {
+                        if (d < dim) {
+                            const double t = xi[r][d] - xj[d];
+                            r2 = __dadd_rn(r2, __dmul_rn(t, t));
+                        }
+                    }
+                    acc[r] = __fma_rn(kernel_value<KIND>(kp, r2), xv, acc[r]);
+                }
             }
         } else {
             for (int jj = 0; jj < cnt; jj++) {

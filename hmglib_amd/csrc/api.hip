@@ -35,23 +35,78 @@ std::vector<LargeBlock> g_large;  // released large buffers, still mapped
 
 namespace {
 constexpr size_t kPinChunk = (size_t)4 << 20;
-// this thread's pinned, device-mapped staging buffer (host and device addresses)
-thread_local void* t_pin = nullptr;
-thread_local void* t_pin_dev = nullptr;
-thread_local size_t t_pin_bytes = 0;
+// Pinned, device-mapped staging buffers (host and device addresses): each thread holds one
+// and hands it on when it ends.  A batched call starts its worker threads anew and each
+// grew a buffer of its own, request by request; hipHostMalloc and hipHostFree wait for the
+// device, and took 150 of 24 clouds' 190 ms.  At most kPinKept (64 MB) wait for another
+// thread; hmg_release_cached_memory returns those.
+struct PinBuf {
+    void* host = nullptr;
+    void* mapped = nullptr;
+    size_t bytes = 0;
+    int dev = 0;
+};
+constexpr size_t kPinKept = 16, kPinMin = (size_t)256 << 10;
+struct PinPool {
+    std::mutex mu;
+    std::vector<PinBuf> free;
+};
+PinPool& pin_pool()
+{
+    static PinPool* p = new PinPool();  // never destroyed: threads may end after it
+    return *p;
+}
+struct PinHolder {
+    PinBuf b;
+    // No call of the runtime here, which may be gone when the process ends; a buffer past
+    // the bound stays with the process as the runtime's
+    ~PinHolder()
+    {
+        if (!b.host) return;
+        PinPool& p = pin_pool();
+        std::lock_guard<std::mutex> lk(p.mu);
+        if (p.free.size() < kPinKept) p.free.push_back(b);
+    }
+};
+thread_local PinHolder t_pin;
+
+void pin_trim()
+{
+    std::vector<PinBuf> out;
+    {
+        std::lock_guard<std::mutex> lk(pin_pool().mu);
+        out.swap(pin_pool().free);
+    }
+    for (const PinBuf& b : out) (void)hipHostFree(b.host);
+}
 
 hmg_status pinned(size_t bytes, void** host, void** dev)
 {
-    if (t_pin_bytes < bytes) {
-        if (t_pin) (void)hipHostFree(t_pin);
-        t_pin = t_pin_dev = nullptr;
-        t_pin_bytes = 0;
-        HMG_HIP(hipHostMalloc(&t_pin, bytes, hipHostMallocMapped | hipHostMallocCoherent));
-        HMG_HIP(hipHostGetDevicePointer(&t_pin_dev, t_pin, 0));
-        t_pin_bytes = bytes;
+    PinBuf& b = t_pin.b;
+    if (!b.host) {
+        int d = 0;
+        HMG_HIP(hipGetDevice(&d));
+        PinPool& p = pin_pool();
+        std::lock_guard<std::mutex> lk(p.mu);
+        for (size_t i = p.free.size(); i-- > 0;) {
+            if (p.free[i].dev != d) continue;
+            b = p.free[i];
+            p.free.erase(p.free.begin() + (ptrdiff_t)i);
+            break;
+        }
     }
-    *host = t_pin;
-    *dev = t_pin_dev;
+    if (b.bytes < bytes) {
+        if (b.host) (void)hipHostFree(b.host);
+        b = PinBuf{};
+        size_t want = kPinMin;
+        while (want < bytes) want *= 2;
+        HMG_HIP(hipGetDevice(&b.dev));
+        HMG_HIP(hipHostMalloc(&b.host, want, hipHostMallocMapped | hipHostMallocCoherent));
+        HMG_HIP(hipHostGetDevicePointer(&b.mapped, b.host, 0));
+        b.bytes = want;
+    }
+    *host = b.host;
+    *dev = b.mapped;
     return HMG_OK;
 }
 
@@ -489,7 +544,11 @@ extern "C" {
 
 const char* hmg_last_error(void) { return g_error.c_str(); }
 
-void hmg_release_cached_memory(void) { large_trim(true); }
+void hmg_release_cached_memory(void)
+{
+    large_trim(true);
+    pin_trim();
+}
 
 // ------------------------------------------------------------------ init
 hmg_status hmg_init_h_matrix_data(struct h_matrix_data* data, int point_count[2], int dim, int bits)

@@ -329,7 +329,9 @@ const char* hmg_last_error(void);
 /* Device buffers of 8 GiB and more (factors, panels, scratch) stay mapped after
  * their H-matrix releases them and are reused by later large allocations on the
  * same device (re-mapping device memory costs about 28 ms per GB on MI355X); this
- * returns them to the devices.  An allocation that fails returns them itself. */
+ * returns them to the devices.  An allocation that fails returns them itself.
+ * Also freed: the pinned staging buffers (4 MiB each, 16 at most) of threads that
+ * have ended. */
 void hmg_release_cached_memory(void);
 /* sizeof / field offsets of the public structs, for FFI layout checks: which =
  * 0 h_matrix_data, 1 work_item, 2 point_set, 3 morton_code, 4 system_assembler,

@@ -447,6 +447,8 @@ void release_build(Engine& e, h_matrix_data* d)
     e.ldu.release();
     e.h_ldu.clear();
     for (Combine* c : {&e.comb_stored, &e.comb_fly}) {
+        c->seg.release();
+        c->row0.release();
         c->ptr.release();
         c->idx.release();
         c->groups.release();
@@ -467,6 +469,8 @@ void release_build(Engine& e, h_matrix_data* d)
     e.n_mx_items = 0;
     e.mx_evals = 0;
     e.mx_sched = false;
+    e.comb_mx.seg.release();
+    e.comb_mx.row0.release();
     e.comb_mx.ptr.release();
     e.comb_mx.idx.release();
     e.comb_mx.groups.release();
@@ -910,8 +914,8 @@ std::vector<const void*> product_state(const h_matrix_data* d, const Engine& e)
 {
     return {d->U, d->V, d->dA, e.U.p, e.V.p, e.Up.p, e.Vp.p, e.A.p, e.keff.p, e.blk.p, e.lr_items.p,
             e.lv_items.p, e.lv_slices.p, e.tmap.p, e.near_items.p, e.near_blk.p, e.fly_items.p, e.fly_refs.p,
-            e.mx_items.p, e.mx_refs.p, e.mx_wg.p, e.vw_items.p, e.uw_items.p, e.comb_stored.idx.p,
-            e.comb_fly.idx.p, e.comb_mx.idx.p, e.xs.p, e.Tp.p, e.T.p, e.P.p, e.X64.p, e.Tp64.p, e.T64.p,
+            e.mx_items.p, e.mx_refs.p, e.mx_wg.p, e.vw_items.p, e.uw_items.p, e.comb_stored.seg.p, e.comb_stored.idx.p,
+            e.comb_fly.seg.p, e.comb_fly.idx.p, e.comb_mx.seg.p, e.comb_mx.idx.p, e.xs.p, e.Tp.p, e.T.p, e.P.p, e.X64.p, e.Tp64.p, e.T64.p,
             e.P64.p, e.Ys64.p, e.inv1.p, e.Xp.p, e.Xt32.p, e.Tpan.p, e.Tp32.p, e.P32.p, e.Ys32.p,
             e.cpan[0].p, e.cpan[1].p, e.mxp.p, d->assem, (const void*)(uintptr_t)e.epoch};
 }
@@ -1229,7 +1233,7 @@ int64_t engine_bytes(const Engine& e)
     t += bytes_of(e.X64) + bytes_of(e.Tp64) + bytes_of(e.T64) + bytes_of(e.P64) + bytes_of(e.Ys64);
     t += bytes_of(e.vw_items) + bytes_of(e.uw_items) + bytes_of(e.mx_wg);
     for (const Combine* c : {&e.comb_stored, &e.comb_fly, &e.comb_mx})
-        t += bytes_of(c->ptr) + bytes_of(c->idx) + bytes_of(c->groups);
+        t += bytes_of(c->seg) + bytes_of(c->row0) + bytes_of(c->ptr) + bytes_of(c->idx) + bytes_of(c->groups);
     return t;
 }
 

@@ -331,12 +331,14 @@ struct MxPanel {
     int pad;
 };
 
-// per-point partial lists of one MVP schedule (CSR over sorted rows): an entry
-// v >= 0 is the P slot v, an entry v < 0 the column-slot group -(v+1)
+// Partial lists of one MVP schedule.  Rows that the same items cover have lists that differ
+// by the row alone: sorted row i lies in segment g = seg[i], which starts at row0[g] and has
+// the list idx[ptr[g], ptr[g + 1]).  An entry v >= 0 is the P slot v + i - row0[g], an entry
+// v < 0 the column-slot group -(v+1).
 struct Combine {
-    DevBuf<int> ptr, idx;
+    DevBuf<int> seg, row0, ptr, idx;
     DevBuf<ColSlots> groups;
-    int64_t total = 0;          // list entries
+    int64_t total = 0;          // list entries of all rows
     int64_t group_entries = 0;  // entries naming a column-slot group
     int64_t slots = 0;          // column slots reached through the groups
 };

@@ -10,7 +10,9 @@
 #include <cstring>
 #include <cstddef>
 
+#include <map>
 #include <mutex>
+#include <new>
 
 #include "hmg_internal.h"
 #include "../../include/hmglib_server.h"
@@ -22,6 +24,7 @@ thread_local std::string g_error;
 }
 
 thread_local hipStream_t g_alloc_stream = nullptr;
+thread_local bool g_alloc_idle = false;
 
 namespace {
 struct LargeBlock {
@@ -231,8 +234,145 @@ void large_free(void* p, size_t held)
     g_large.push_back(LargeBlock{dev, p, held});
 }
 
+namespace {
+struct IdleBlock {
+    void* p;
+    uint64_t age;
+};
+struct IdlePool {
+    std::mutex mu;
+    std::multimap<std::pair<int, size_t>, IdleBlock> blocks;  // by device and bytes
+    size_t bytes = 0;
+    uint64_t puts = 0;
+    std::vector<std::pair<int, hipStream_t>> streams;
+};
+IdlePool& idle_pool()
+{
+    static IdlePool* p = new IdlePool();  // never destroyed: see pin_pool
+    return *p;
+}
+// small ones are cheap in the device's pool
+constexpr size_t kIdleMin = (size_t)4 << 10;
+constexpr size_t kIdleBlocks = 4096, kIdleStreams = 64;
+}  // namespace
+
+void* idle_take(size_t bytes, hipStream_t s, size_t* size)
+{
+    int dev = 0;
+    if (bytes < kIdleMin || hipStreamGetDevice(s, &dev) != hipSuccess) return nullptr;
+    IdlePool& pool = idle_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    const auto it = pool.blocks.lower_bound({dev, bytes});
+    if (it == pool.blocks.end() || it->first.first != dev || it->first.second > bytes + bytes / 4) return nullptr;
+    void* p = it->second.p;
+    *size = it->first.second;
+    pool.bytes -= *size;
+    pool.blocks.erase(it);
+    return p;
+}
+
+void idle_put(void* p, size_t size, hipStream_t s)
+{
+    int dev = 0;
+    if (size < kIdleMin || size > kIdleBytes || hipStreamGetDevice(s, &dev) != hipSuccess) {
+        (void)hipFreeAsync(p, s);
+        return;
+    }
+    void* out = p;
+    try {
+        IdlePool& pool = idle_pool();
+        std::lock_guard<std::mutex> lk(pool.mu);
+        if (pool.bytes + size > kIdleBytes || pool.blocks.size() >= kIdleBlocks) {
+            // the oldest that makes room goes for it
+            auto old = pool.blocks.end();
+            for (auto it = pool.blocks.lower_bound({dev, 0}); it != pool.blocks.end() && it->first.first == dev; ++it)
+                if (pool.bytes - it->first.second + size <= kIdleBytes &&
+                    (old == pool.blocks.end() || it->second.age < old->second.age))
+                    old = it;
+            if (old != pool.blocks.end()) {
+                const IdleBlock b = old->second;
+                const size_t n = old->first.second;
+                pool.blocks.emplace(std::make_pair(dev, size), IdleBlock{p, pool.puts++});
+                pool.blocks.erase(old);
+                pool.bytes += size - n;
+                out = b.p;
+            }
+        } else {
+            pool.blocks.emplace(std::make_pair(dev, size), IdleBlock{p, pool.puts++});
+            pool.bytes += size;
+            out = nullptr;
+        }
+    } catch (const std::bad_alloc&) {
+    }
+    if (out) (void)hipFreeAsync(out, s);
+}
+
+void idle_trim(bool every)
+{
+    int cur = 0;
+    if (hipGetDevice(&cur) != hipSuccess) return;
+    std::multimap<std::pair<int, size_t>, IdleBlock> out;
+    {
+        IdlePool& pool = idle_pool();
+        std::lock_guard<std::mutex> lk(pool.mu);
+        for (auto it = pool.blocks.begin(); it != pool.blocks.end();) {
+            const auto at = it++;
+            if (!every && at->first.first != cur) continue;
+            pool.bytes -= at->first.second;
+            out.insert(pool.blocks.extract(at));
+        }
+    }
+    for (auto it = out.begin(); it != out.end();) {
+        const int dev = it->first.first;
+        if (dev != cur) (void)hipSetDevice(dev);
+        for (; it != out.end() && it->first.first == dev; ++it) (void)hipFreeAsync(it->second.p, nullptr);
+        hipMemPool_t mp = nullptr;
+        if (hipDeviceSynchronize() == hipSuccess && hipDeviceGetDefaultMemPool(&mp, dev) == hipSuccess)
+            (void)hipMemPoolTrimTo(mp, 0);
+        if (dev != cur) (void)hipSetDevice(cur);
+    }
+}
+
+hmg_status stream_take(hipStream_t* out)
+{
+    int dev = 0;
+    HMG_HIP(hipGetDevice(&dev));
+    {
+        IdlePool& pool = idle_pool();
+        std::lock_guard<std::mutex> lk(pool.mu);
+        for (auto it = pool.streams.begin(); it != pool.streams.end(); ++it) {
+            if (it->first != dev) continue;
+            *out = it->second;
+            pool.streams.erase(it);
+            return HMG_OK;
+        }
+    }
+    HMG_HIP(hipStreamCreateWithFlags(out, hipStreamNonBlocking));
+    return HMG_OK;
+}
+
+void stream_put(hipStream_t s)
+{
+    int dev = 0;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusActive;
+    if (hipStreamSynchronize(s) == hipSuccess && hipStreamIsCapturing(s, &cap) == hipSuccess &&
+        cap == hipStreamCaptureStatusNone && hipStreamGetDevice(s, &dev) == hipSuccess) {
+        try {
+            IdlePool& pool = idle_pool();
+            std::lock_guard<std::mutex> lk(pool.mu);
+            if (pool.streams.size() < kIdleStreams) {
+                pool.streams.emplace_back(dev, s);
+                return;
+            }
+        } catch (const std::bad_alloc&) {
+        }
+    }
+    (void)hipStreamDestroy(s);
+}
+
 void reclaim_device_memory()
 {
+    idle_trim(false);
     large_trim(false);
     int dev = 0;
     hipMemPool_t pool = nullptr;
@@ -550,6 +690,7 @@ const char* hmg_last_error(void) { return g_error.c_str(); }
 
 void hmg_release_cached_memory(void)
 {
+    idle_trim(true);
     large_trim(true);
     pin_trim();
 }
@@ -596,8 +737,8 @@ hmg_status engine_init(h_matrix_data* data, int point_count[2], int dim, int bit
     } else {
         // non-blocking streams: no implicit ordering with the null stream, so the
         // work of independent H-matrices driven from different host threads overlaps
-        HMG_HIP(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
-        HMG_HIP(hipStreamCreateWithFlags(&e->stream2, hipStreamNonBlocking));
+        HMG_TRY(stream_take(&e->stream));
+        HMG_TRY(stream_take(&e->stream2));
     }
     HMG_HIP(hipEventCreateWithFlags(&e->ev_fork, hipEventDisableTiming));
     HMG_HIP(hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming));
@@ -875,6 +1016,10 @@ hmg_status hmg_precompute_dense(struct h_matrix_data* data)
     size_t free_b = 0, total_b = 0;
     HMG_HIP(hipMemGetInfo(&free_b, &total_b));
     const double need = 8.0 * (double)entries;
+    if (need > (double)free_b * 0.95) {
+        idle_trim(false);  // kept buffers don't refuse it
+        HMG_HIP(hipMemGetInfo(&free_b, &total_b));
+    }
     if (need > (double)free_b * 0.95) {
         set_error("dense blocks need " + std::to_string(need / 1e9) + " GB but only " +
                   std::to_string(free_b / 1e9) + " GB of device memory are free; "
@@ -1459,6 +1604,7 @@ hmg_status hmg_destroy_h_matrix_data(struct h_matrix_data* data)
         (void)hipStreamSynchronize(e->stream);
     }
     hipStream_t s = e->stream;
+    IdleScope idle(e->own_streams);
     {
         AllocScope scope(s);
         release_build(*e, data);
@@ -1504,10 +1650,8 @@ hmg_status hmg_destroy_h_matrix_data(struct h_matrix_data* data)
     data->engine = nullptr;
     data->magma_queue = nullptr;
     if (own) {
-        (void)hipStreamSynchronize(st2);
-        (void)hipStreamSynchronize(st);
-        (void)hipStreamDestroy(st2);
-        (void)hipStreamDestroy(st);
+        stream_put(st2);
+        stream_put(st);
     }
     return HMG_OK;
 }

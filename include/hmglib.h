@@ -330,7 +330,8 @@ const char* hmg_last_error(void);
  * their H-matrix releases them and are reused by later large allocations on the
  * same device (re-mapping device memory costs about 28 ms per GB on MI355X); this
  * returns them to the devices.  An allocation that fails returns them itself.
- * Also freed: the pinned staging buffers (4 MiB each, 16 at most) of threads that
+ * Also returned: up to 4 GiB of smaller buffers of destroyed H-matrices, kept for
+ * later ones, and the pinned staging buffers (4 MiB each, 16 at most) of threads that
  * have ended. */
 void hmg_release_cached_memory(void);
 /* sizeof / field offsets of the public structs, for FFI layout checks: which =

@@ -1128,6 +1128,7 @@ hmg_status aca_build_mixed(Engine& eng, const Coords& c1, const Coords& c2, cons
         used += need;
     }
     const int nb = (int)members.size();
+    IdleScope idle(false);  // outlives the scratch
     DevBuf<double> S;
     HMG_TRY(S.alloc((size_t)scratch));
     DevBuf<int64_t> d_suoff, d_svoff;
@@ -1161,6 +1162,7 @@ hmg_status aca_build_mixed(Engine& eng, const Coords& c1, const Coords& c2, cons
     }
     eng.prof.end(PROF_ACA, s);
     HMG_HIP(hipStreamSynchronize(s));
+    g_alloc_idle = eng.own_streams;  // nothing uses the scratch any more
     return HMG_OK;
 }
 

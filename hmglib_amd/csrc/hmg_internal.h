@@ -110,6 +110,14 @@ struct IdleScope {
     IdleScope(const IdleScope&) = delete;
     IdleScope& operator=(const IdleScope&) = delete;
 };
+// bytes to ask the pool for: up to the next sixteenth of an octave, so that the buffers of
+// another cloud of the same size serve
+inline size_t idle_size(size_t bytes)
+{
+    size_t q = 1;
+    while (bytes / q >= 32) q *= 2;
+    return bytes < 4096 ? bytes : (bytes + q - 1) / q * q;
+}
 // a kept buffer for `bytes` on the stream's device (its size in *size), or nullptr
 void* idle_take(size_t bytes, hipStream_t s, size_t* size);
 // keeps p, which no work uses any more; `s`, a stream of its device, frees what has to go for it
@@ -166,9 +174,9 @@ struct DevBuf {
             e = large_alloc((void**)&p, bytes, &held);
         } else {
             st = g_alloc_stream;
-            size = bytes;
+            size = st ? idle_size(bytes) : bytes;
             p = st ? (T*)idle_take(bytes, st, &size) : nullptr;
-            e = p ? hipSuccess : st ? hipMallocAsync((void**)&p, bytes, st) : hipMalloc(&p, bytes);
+            e = p ? hipSuccess : st ? hipMallocAsync((void**)&p, size, st) : hipMalloc(&p, bytes);
             if (e != hipSuccess) {
                 // cached large buffers or the pool may hold the memory: return it and retry
                 (void)hipGetLastError();

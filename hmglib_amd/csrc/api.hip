@@ -239,18 +239,11 @@ struct IdleBlock {
     void* p;
     uint64_t age;
 };
-// an H-matrix' two streams stay together: made one after the other, they have hardware
-// queues of their own
-struct StreamPair {
-    int dev;
-    hipStream_t s1, s2;
-};
 struct IdlePool {
     std::mutex mu;
     std::multimap<std::pair<int, size_t>, IdleBlock> blocks;  // by device and bytes
     size_t bytes = 0;
     uint64_t puts = 0;
-    std::vector<StreamPair> streams;
 };
 IdlePool& idle_pool()
 {
@@ -259,7 +252,7 @@ IdlePool& idle_pool()
 }
 // small ones are cheap in the device's pool
 constexpr size_t kIdleMin = (size_t)4 << 10;
-constexpr size_t kIdleBlocks = 4096, kIdlePairs = 32;
+constexpr size_t kIdleBlocks = 4096;
 }  // namespace
 
 void* idle_take(size_t bytes, hipStream_t s, size_t* size)
@@ -337,50 +330,6 @@ void idle_trim(bool every)
             (void)hipMemPoolTrimTo(mp, 0);
         if (dev != cur) (void)hipSetDevice(cur);
     }
-}
-
-hmg_status stream_take(hipStream_t* s1, hipStream_t* s2)
-{
-    int dev = 0;
-    HMG_HIP(hipGetDevice(&dev));
-    {
-        IdlePool& pool = idle_pool();
-        std::lock_guard<std::mutex> lk(pool.mu);
-        for (auto it = pool.streams.begin(); it != pool.streams.end(); ++it) {
-            if (it->dev != dev) continue;
-            *s1 = it->s1;
-            *s2 = it->s2;
-            pool.streams.erase(it);
-            return HMG_OK;
-        }
-    }
-    HMG_HIP(hipStreamCreateWithFlags(s1, hipStreamNonBlocking));
-    HMG_HIP(hipStreamCreateWithFlags(s2, hipStreamNonBlocking));
-    return HMG_OK;
-}
-
-void stream_put(hipStream_t s1, hipStream_t s2)
-{
-    auto idle = [](hipStream_t s) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusActive;
-        return hipStreamSynchronize(s) == hipSuccess && hipStreamIsCapturing(s, &cap) == hipSuccess &&
-               cap == hipStreamCaptureStatusNone;
-    };
-    int dev = 0;
-    const bool idle2 = idle(s2), idle1 = idle(s1);
-    if (idle1 && idle2 && hipStreamGetDevice(s1, &dev) == hipSuccess) {
-        try {
-            IdlePool& pool = idle_pool();
-            std::lock_guard<std::mutex> lk(pool.mu);
-            if (pool.streams.size() < kIdlePairs) {
-                pool.streams.push_back(StreamPair{dev, s1, s2});
-                return;
-            }
-        } catch (const std::bad_alloc&) {
-        }
-    }
-    (void)hipStreamDestroy(s2);
-    (void)hipStreamDestroy(s1);
 }
 
 void reclaim_device_memory()
@@ -750,7 +699,8 @@ hmg_status engine_init(h_matrix_data* data, int point_count[2], int dim, int bit
     } else {
         // non-blocking streams: no implicit ordering with the null stream, so the
         // work of independent H-matrices driven from different host threads overlaps
-        HMG_TRY(stream_take(&e->stream, &e->stream2));
+        HMG_HIP(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
+        HMG_HIP(hipStreamCreateWithFlags(&e->stream2, hipStreamNonBlocking));
     }
     HMG_HIP(hipEventCreateWithFlags(&e->ev_fork, hipEventDisableTiming));
     HMG_HIP(hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming));
@@ -1662,7 +1612,10 @@ hmg_status hmg_destroy_h_matrix_data(struct h_matrix_data* data)
     data->engine = nullptr;
     data->magma_queue = nullptr;
     if (own) {
-        stream_put(st, st2);
+        (void)hipStreamSynchronize(st2);
+        (void)hipStreamSynchronize(st);
+        (void)hipStreamDestroy(st2);
+        (void)hipStreamDestroy(st);
     }
     return HMG_OK;
 }

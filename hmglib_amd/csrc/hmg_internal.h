@@ -100,7 +100,8 @@ void reclaim_device_memory();
 // of destroying 24 clouds.  A buffer serves a request of at least four fifths of its size on its device.
 // At most kIdleBytes stay, the oldest go first; an allocation that fails and
 // hmg_release_cached_memory return them all.  Set on the thread that destroys
-// (IdleScope): releases go there.  Their pairs of streams are kept too, 32 at most (0.9 ms for new ones).
+// (IdleScope): releases go there.  (Streams are made anew: kept
+// ones, whose hardware queues then never change, made products 6 to 9 % slower.)
 constexpr size_t kIdleBytes = (size_t)4 << 30;
 extern thread_local bool g_alloc_idle;
 struct IdleScope {
@@ -124,8 +125,6 @@ void* idle_take(size_t bytes, hipStream_t s, size_t* size);
 void idle_put(void* p, size_t size, hipStream_t s);
 // returns the kept buffers of the current device (all devices: every = true)
 void idle_trim(bool every);
-hmg_status stream_take(hipStream_t* s1, hipStream_t* s2);
-void stream_put(hipStream_t s1, hipStream_t s2);
 
 template <class T>
 struct DevBuf {

@@ -1,4 +1,4 @@
-"""Buffers and streams kept from destroyed H-matrices: products of H-matrices built in
+"""Buffers kept from destroyed H-matrices: products of H-matrices built in
 them, by several threads and after giving everything back, are bitwise those of the first
 build; the bytes kept stay bounded."""
 import threading

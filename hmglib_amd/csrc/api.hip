@@ -3,6 +3,7 @@
 // Host orchestration only; every computation runs in the HIP kernels of
 // prims/morton/tree/aca/mvp.hip on the engine's stream.  All calls are
 // synchronous, as in the reference.
+#include <atomic>
 #include <chrono>
 #include <climits>
 #include <cmath>
@@ -366,6 +367,12 @@ void large_trim(bool every)
 
 void set_error(const std::string& msg) { g_error = msg; }
 
+uint64_t next_epoch()
+{
+    static std::atomic<uint64_t> last{0};
+    return ++last;
+}
+
 Engine* engine_of(const h_matrix_data* d) { return d ? (Engine*)d->engine : nullptr; }
 
 void Profiler::begin(int cls, hipStream_t s)
@@ -487,7 +494,7 @@ int aca_work_size_at(const std::vector<int4>& bl, int nblocks, int64_t max_size,
 
 void release_factors(Engine& e, h_matrix_data* d)
 {
-    e.epoch++;
+    e.epoch = next_epoch();
     e.U.release();
     e.V.release();
     e.Up.release();
@@ -879,7 +886,7 @@ void release_build_state(Engine& e, h_matrix_data* d) { release_build(e, d); }
 hmg_status finish_setup(h_matrix_data* data, Engine* e)
 {
     AllocScope scope(e->stream);
-    e->epoch++;
+    e->epoch = next_epoch();
     data->mat_vec_data = (work_item**)malloc(sizeof(work_item*));
     *data->mat_vec_data = e->blocks.p;
     data->mat_vec_data_count = e->nblocks;
@@ -959,7 +966,7 @@ hmg_status hmg_precompute_aca(struct h_matrix_data* data)
         data->V = e->V.p;
     }
     e->fact_prec = e->precision;
-    e->epoch++;
+    e->epoch = next_epoch();
     return HMG_OK;
 }
 
@@ -1424,7 +1431,7 @@ hmg_status hmg_set_option(struct h_matrix_data* data, int option, int64_t value)
         set_error("h_matrix_data not initialised");
         return HMG_ERR_NOT_READY;
     }
-    e->epoch++;
+    e->epoch = next_epoch();
     switch (option) {
     case HMG_OPT_NEAR_SYMMETRIC:
         e->near_sym_enabled = value != 0;

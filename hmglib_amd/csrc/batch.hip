@@ -696,7 +696,7 @@ extern "C" hmg_status hmg_precompute_aca_batch(struct h_matrix_data* const* data
             data[i]->V = e->V.p;
         }
         e->fact_prec = e->precision;
-        e->epoch++;
+        e->epoch = next_epoch();
     }
     return HMG_OK;
 }

@@ -382,6 +382,9 @@ struct Combine {
     int64_t slots = 0;          // column slots reached through the groups
 };
 
+// a number that no earlier call in the process returned
+uint64_t next_epoch();
+
 // ---- engine state hung off h_matrix_data::engine ---------------------------
 struct Engine {
     Profiler prof;
@@ -390,7 +393,10 @@ struct Engine {
     int dim = 0;
     int bits = 0;
     bool built = false;
-    uint64_t epoch = 0;  // bumped by every change of set-up, factors or options
+    // new at every change of set-up, factors or options, and no other engine's, before or
+    // after: a captured product of a destroyed H-matrix is told from one of its successor,
+    // which may stand in the same struct and the same buffers
+    uint64_t epoch = next_epoch();
 
     DevBuf<uint32_t> perm32[2];                 // sort values
     DevBuf<work_item> blocks;                   // final block list (DENSE first)

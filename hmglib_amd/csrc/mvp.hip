@@ -607,7 +607,7 @@ hmg_status dense_fill(Engine& eng, const Coords& c1, const Coords& c2, const Ker
     }
     HMG_HIP(hipStreamSynchronize(s));
     eng.dense_stored = true;
-    eng.epoch++;
+    eng.epoch = next_epoch();
     return HMG_OK;
 }
 

@@ -730,7 +730,12 @@ aca_reg_kernel(AcaArgs g)
 // thread at a time with eight terms of each in flight.  The slab is written to V_b at the end.
 // Bound by those reads (ranks^2 / 2 terms per row, past the L2 for many blocks at once):
 // about 9 TB/s at N = 262144 in 3D, 22 ms of that build.
+// Sums over columns or rows are formed as a team of kWideWaves wavefronts forms them (one
+// partial sum per thread of such a team, reduced per wavefront, added in order), whatever
+// NW: a smaller team holds several of its threads' sums.  A block's ranks and factors then
+// do not depend on the team that the launch chose.
 constexpr int kWideCols = 4;
+constexpr int kWideWaves = 8;
 
 // val[e] -= sum_{l < r} s[l] p[l * sp + off[e]] in l order
 __device__ __forceinline__ void wide_chain(double (&val)[kWideCols], const double* s, int r, const double* p, int64_t sp,
@@ -755,9 +760,11 @@ __device__ __forceinline__ void wide_chain(double (&val)[kWideCols], const doubl
 }
 
 template <int KIND, int DIM, bool TOL, int NW>
-__device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegShared<NW, DIM>& sh, double* vt)
+__device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegShared<kWideWaves, DIM>& sh, double* vt)
 {
     constexpr int TS = NW * kWave, E = kWideCols;
+    constexpr int H = kWideWaves / NW;  // partial sums per thread: element i belongs to sum i / TS % H
+    static_assert(H * NW == kWideWaves && E % H == 0, "whole wavefronts");
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int lane = threadIdx.x % kWave;
@@ -779,12 +786,15 @@ __device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegSha
         __syncthreads();
         return t;
     };
-    auto team_sum = [&](double v) {
-        v = wave_add(v);
-        if (lane == 0) sh.ext[w] = v;
+    auto team_sum = [&](const double (&v)[H]) {
+#pragma unroll
+        for (int h = 0; h < H; h++) {
+            const double x = wave_add(v[h]);
+            if (lane == 0) sh.ext[h * NW + w] = x;
+        }
         __syncthreads();
         double t = 0.0;
-        for (int q = 0; q < NW; q++) t += sh.ext[q];
+        for (int q = 0; q < kWideWaves; q++) t += sh.ext[q];
         __syncthreads();
         return t;
     };
@@ -866,7 +876,7 @@ __device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegSha
             if (tid < r) sh.u[tid] = Ub[tid * lu + i_r];
             if (tid >= kRegRank && tid < kRegRank + DIM) sh.xu[tid - kRegRank] = g.c1.x[tid - kRegRank][l1 + i_r];
             __syncthreads();
-            double nw = 0.0, best = -1.0, bval = 0.0;
+            double nw[H] = {0.0}, best = -1.0, bval = 0.0;
             int bj = -1;
             for (int j0 = tid; j0 < m2; j0 += E * TS) {
                 int off[E];
@@ -886,7 +896,7 @@ __device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegSha
                     const int j = j0 + e * TS;
                     if (j < m2) {
                         vt[r * vs + j] = val[e];
-                        nw = __fma_rn(val[e], val[e], nw);
+                        nw[e % H] = __fma_rn(val[e], val[e], nw[e % H]);
                         const double ax = fabs(val[e]);
                         if (g.tie_last ? ax >= best : ax > best) {
                             best = ax;
@@ -896,7 +906,8 @@ __device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegSha
                     }
                 }
             }
-            nw = wave_add(nw);
+#pragma unroll
+            for (int h = 0; h < H; h++) nw[h] = wave_add(nw[h]);
             const double wb = wave_max(best);
             uint64_t mask = __ballot(best == wb);
             if (mask & (mask - 1)) {  // equal candidates: the last (first) index
@@ -908,14 +919,15 @@ __device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegSha
             const int wj = __builtin_amdgcn_readlane(bj, wl);
             const double wv = lane_of(bval, wl);
             if (lane == 0) {
-                sh.red[w] = nw;
+#pragma unroll
+                for (int h = 0; h < H; h++) sh.red[h * NW + w] = nw[h];
                 sh.best[w] = wb;
                 sh.bval[w] = wv;
                 sh.bj[w] = wj;
             }
             __syncthreads();
             double nrm = 0.0;
-            for (int q = 0; q < NW; q++) nrm += sh.red[q];
+            for (int q = 0; q < kWideWaves; q++) nrm += sh.red[q];
             double bb = sh.best[0];
             jr = sh.bj[0];
             p = sh.bval[0];
@@ -941,43 +953,45 @@ __device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegSha
             if (n > 0 && tid < kRegAhead * DIM)
                 sh.tx[tid / DIM][tid % DIM] = g.c1.x[tid % DIM][l1 + i_r + 1 + min(tid / DIM, n - 1)];
             __syncthreads();
-            double tn[kRegAhead];
+            for (int h = 0; h < H; h++) {
+                double tn[kRegAhead];
 #pragma unroll
-            for (int e = 0; e < kRegAhead; e++) tn[e] = 0.0;
-            for (int j = n > 0 ? tid : m2; j < m2; j += TS) {
-                double y[DIM], t[kRegAhead];
+                for (int e = 0; e < kRegAhead; e++) tn[e] = 0.0;
+                for (int j = n > 0 ? tid + h * TS : m2; j < m2; j += H * TS) {
+                    double y[DIM], t[kRegAhead];
 #pragma unroll
-                for (int d = 0; d < DIM; d++) y[d] = g.c2.x[d][l2 + j];
+                    for (int d = 0; d < DIM; d++) y[d] = g.c2.x[d][l2 + j];
 #pragma unroll
-                for (int e = 0; e < kRegAhead; e++) t[e] = entry(sh.tx[e], y, l1 + i_r + 1 + e, l2 + j);
-                int l = 0;
-                for (; l + 8 <= r; l += 8) {
-                    double x[8];
+                    for (int e = 0; e < kRegAhead; e++) t[e] = entry(sh.tx[e], y, l1 + i_r + 1 + e, l2 + j);
+                    int l = 0;
+                    for (; l + 8 <= r; l += 8) {
+                        double x[8];
 #pragma unroll
-                    for (int q = 0; q < 8; q++) x[q] = vt[(l + q) * vs + j];
+                        for (int q = 0; q < 8; q++) x[q] = vt[(l + q) * vs + j];
 #pragma unroll
-                    for (int q = 0; q < 8; q++)
+                        for (int q = 0; q < 8; q++)
 #pragma unroll
-                        for (int e = 0; e < kRegAhead; e++) t[e] = __fma_rn(-sh.tu[e][l + q], x[q], t[e]);
+                            for (int e = 0; e < kRegAhead; e++) t[e] = __fma_rn(-sh.tu[e][l + q], x[q], t[e]);
+                    }
+                    for (; l < r; l++) {
+                        const double x = vt[l * vs + j];
+#pragma unroll
+                        for (int e = 0; e < kRegAhead; e++) t[e] = __fma_rn(-sh.tu[e][l], x, t[e]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < kRegAhead; e++) tn[e] = __fma_rn(t[e], t[e], tn[e]);
                 }
-                for (; l < r; l++) {
-                    const double x = vt[l * vs + j];
 #pragma unroll
-                    for (int e = 0; e < kRegAhead; e++) t[e] = __fma_rn(-sh.tu[e][l], x, t[e]);
+                for (int e = 0; e < kRegAhead; e++) {
+                    tn[e] = wave_add(tn[e]);
+                    if (lane == 0) sh.tn[e][h * NW + w] = tn[e];
                 }
-#pragma unroll
-                for (int e = 0; e < kRegAhead; e++) tn[e] = __fma_rn(t[e], t[e], tn[e]);
-            }
-#pragma unroll
-            for (int e = 0; e < kRegAhead; e++) {
-                tn[e] = wave_add(tn[e]);
-                if (lane == 0) sh.tn[e][w] = tn[e];
             }
             __syncthreads();
             int skip = 0;
             for (; skip < n; skip++) {
                 double t = 0.0;
-                for (int q = 0; q < NW; q++) t += sh.tn[skip][q];
+                for (int q = 0; q < kWideWaves; q++) t += sh.tn[skip][q];
                 if (sqrt(lane_of(t, 0)) >= 1.0e-13) break;
             }
             i_r += skip;
@@ -993,11 +1007,17 @@ __device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegSha
         if (tid < r) sh.v[tid] = vt[tid * vs + jr];
         if (tid >= kRegRank && tid < kRegRank + DIM) sh.xv[tid - kRegRank] = g.c2.x[tid - kRegRank][l2 + jr];
         __syncthreads();
-        double nu = 0.0, nv = 0.0;
-        for (int j = tid; j < m2; j += TS) {
-            const double x = vt[r * vs + j] / p;
-            vt[r * vs + j] = x;
-            if (TOL) nv = __fma_rn(x, x, nv);
+        double nu[H] = {0.0}, nv[H] = {0.0};
+        for (int j0 = tid; j0 < m2; j0 += H * TS) {
+#pragma unroll
+            for (int h = 0; h < H; h++) {
+                const int j = j0 + h * TS;
+                if (j < m2) {
+                    const double x = vt[r * vs + j] / p;
+                    vt[r * vs + j] = x;
+                    if (TOL) nv[h] = __fma_rn(x, x, nv[h]);
+                }
+            }
         }
         for (int i0 = tid; i0 < m1; i0 += E * TS) {
             int off[E];
@@ -1016,18 +1036,19 @@ __device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegSha
             for (int e = 0; e < E; e++) {
                 if (i0 + e * TS < m1) {
                     Ub[r * lu + i0 + e * TS] = val[e];
-                    if (TOL) nu = __fma_rn(val[e], val[e], nu);
+                    if (TOL) nu[e % H] = __fma_rn(val[e], val[e], nu[e % H]);
                 }
             }
         }
         ke = r + 1;
         if (TOL) {
             // ||U V^T||_F^2 gains 2 u_r . (U (V^T v_r)) + ||u_r||^2 ||v_r||^2
-            for (int q0 = 0; q0 < r; q0 += 8) {
+            for (int c = 0; c < (r + 7) / 8 * H; c++) {
+                const int q0 = c / H * 8, h = c % H;
                 double q[8];
 #pragma unroll
                 for (int e = 0; e < 8; e++) q[e] = 0.0;
-                for (int j = tid; j < m2; j += TS) {
+                for (int j = tid + h * TS; j < m2; j += H * TS) {
                     const double x = vt[r * vs + j];
 #pragma unroll
                     for (int e = 0; e < 8; e++)
@@ -1036,17 +1057,17 @@ __device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegSha
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
                     q[e] = wave_add(q[e]);
-                    if (lane == 0) sh.g[w][q0 + e] = q[e];
+                    if (lane == 0) sh.g[h * NW + w][q0 + e] = q[e];
                 }
             }
             __syncthreads();
             if (tid < r) {
                 double x = 0.0;
-                for (int q = 0; q < NW; q++) x += sh.g[q][tid];
+                for (int q = 0; q < kWideWaves; q++) x += sh.g[q][tid];
                 sh.v[tid] = -x;
             }
             __syncthreads();
-            double cross = 0.0;
+            double cross[H] = {0.0};
             for (int i0 = tid; i0 < m1; i0 += E * TS) {
                 int off[E];
                 double val[E];
@@ -1058,13 +1079,11 @@ __device__ __forceinline__ void wide_block(const AcaArgs& g, const int a, RegSha
                 wide_chain(val, sh.v, r, Ub, lu, off);
 #pragma unroll
                 for (int e = 0; e < E; e++)
-                    if (i0 + e * TS < m1) cross = __fma_rn(val[e], Ub[r * lu + i0 + e * TS], cross);
+                    if (i0 + e * TS < m1) cross[e % H] = __fma_rn(val[e], Ub[r * lu + i0 + e * TS], cross[e % H]);
             }
-            nu = team_sum(nu);
-            nv = team_sum(nv);
-            cross = team_sum(cross);
-            fro2 = fro2 + 2.0 * cross + nu * nv;
-            const bool m = (g.tol.mode == 2 || r % 5 == 0) && sqrt(nu) * sqrt(nv) <= g.tol.c * sqrt(fmax(fro2, 0.0));
+            const double su = team_sum(nu), sv = team_sum(nv);
+            fro2 = fro2 + 2.0 * team_sum(cross) + su * sv;
+            const bool m = (g.tol.mode == 2 || r % 5 == 0) && sqrt(su) * sqrt(sv) <= g.tol.c * sqrt(fmax(fro2, 0.0));
             met = __builtin_amdgcn_readfirstlane(m ? 1 : 0) != 0;
         }
     }
@@ -1087,7 +1106,7 @@ template <int KIND, int DIM, bool TOL, int NW>
 __global__ void __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(3, 3)))
 aca_wide_kernel(AcaArgs g)
 {
-    __shared__ RegShared<NW, DIM> sh;
+    __shared__ RegShared<kWideWaves, DIM> sh;
     const int n = g.resume ? *g.count : g.nlist;
     double* const vt = g.slabs + (int64_t)blockIdx.x * g.slab;
     for (;;) {

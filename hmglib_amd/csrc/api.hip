@@ -556,9 +556,7 @@ void release_build(Engine& e, h_matrix_data* d)
     e.ldu.release();
     e.h_ldu.clear();
     for (Combine* c : {&e.comb_stored, &e.comb_fly}) {
-        c->seg.release();
-        c->row0.release();
-        c->ptr.release();
+        c->rows.release();
         c->idx.release();
         c->groups.release();
         c->total = 0;
@@ -578,9 +576,7 @@ void release_build(Engine& e, h_matrix_data* d)
     e.n_mx_items = 0;
     e.mx_evals = 0;
     e.mx_sched = false;
-    e.comb_mx.seg.release();
-    e.comb_mx.row0.release();
-    e.comb_mx.ptr.release();
+    e.comb_mx.rows.release();
     e.comb_mx.idx.release();
     e.comb_mx.groups.release();
     e.comb_mx.total = 0;
@@ -1028,8 +1024,8 @@ std::vector<const void*> product_state(const h_matrix_data* d, const Engine& e)
 {
     return {d->U, d->V, d->dA, e.U.p, e.V.p, e.Up.p, e.Vp.p, e.A.p, e.keff.p, e.blk.p, e.lr_items.p,
             e.lv_items.p, e.lv_slices.p, e.tmap.p, e.near_items.p, e.near_blk.p, e.fly_items.p, e.fly_refs.p,
-            e.mx_items.p, e.mx_refs.p, e.mx_wg.p, e.vw_items.p, e.uw_items.p, e.comb_stored.seg.p, e.comb_stored.idx.p,
-            e.comb_fly.seg.p, e.comb_fly.idx.p, e.comb_mx.seg.p, e.comb_mx.idx.p, e.xs.p, e.Tp.p, e.T.p, e.P.p, e.X64.p, e.Tp64.p, e.T64.p,
+            e.mx_items.p, e.mx_refs.p, e.mx_wg.p, e.vw_items.p, e.uw_items.p, e.comb_stored.rows.p, e.comb_stored.idx.p,
+            e.comb_fly.rows.p, e.comb_fly.idx.p, e.comb_mx.rows.p, e.comb_mx.idx.p, e.xs.p, e.Tp.p, e.T.p, e.P.p, e.X64.p, e.Tp64.p, e.T64.p,
             e.P64.p, e.Ys64.p, e.inv1.p, e.Xp.p, e.Xt32.p, e.Tpan.p, e.Tp32.p, e.P32.p, e.Ys32.p,
             e.cpan[0].p, e.cpan[1].p, e.mxp.p, d->assem, (const void*)(uintptr_t)e.epoch};
 }
@@ -1347,7 +1343,7 @@ int64_t engine_bytes(const Engine& e)
     t += bytes_of(e.X64) + bytes_of(e.Tp64) + bytes_of(e.T64) + bytes_of(e.P64) + bytes_of(e.Ys64);
     t += bytes_of(e.vw_items) + bytes_of(e.uw_items) + bytes_of(e.mx_wg);
     for (const Combine* c : {&e.comb_stored, &e.comb_fly, &e.comb_mx})
-        t += bytes_of(c->seg) + bytes_of(c->row0) + bytes_of(c->ptr) + bytes_of(c->idx) + bytes_of(c->groups);
+        t += bytes_of(c->rows) + bytes_of(c->idx) + bytes_of(c->groups);
     return t;
 }
 
@@ -1409,7 +1405,7 @@ hmg_status hmg_memory(const struct h_matrix_data* data, int64_t out[2])
         const int64_t slots = (int64_t)e->n_lr_items * 64 + mx_items * 128;
         add += g2 * 2 * kMxRhs * 8 * 2 + (int64_t)e->n[1] * kMxRhs * 4;         // Xp, Xt32
         add += (e->tsize + 32 * (int64_t)ncg) * kMxRhs * 4 + ntp * kMxVCols * kMxRhs * 4;  // Tpan, Tp32
-        add += slots * kMxRhs * 4 + slots * 4 + n1 * 4;              // P32, combine list
+        add += slots * kMxRhs * 4 + slots * 4 + n1 * 16;             // P32, combine list
         add += n1 * kMxRhs * 4 + n1 * 4;                             // Ys32, inv1
         add += (g1 + g2) * e->dim * 8 * 4 + mx_items * (16 + 16);    // panels, items
     }

@@ -371,11 +371,12 @@ struct MxPanel {
 };
 
 // Partial lists of one MVP schedule.  Rows that the same items cover have lists that differ
-// by the row alone: sorted row i lies in segment g = seg[i], which starts at row0[g] and has
-// the list idx[ptr[g], ptr[g + 1]).  An entry v >= 0 is the P slot v + i - row0[g], an entry
-// v < 0 the column-slot group -(v+1).
+// by the row alone: sorted row i with rows[i] = {q0, q1, o, 0} has the list idx[q0, q1), the
+// list of its segment of rows, o rows past whose first one it lies.  An entry v >= 0 is the
+// P slot v + o, an entry v < 0 the column-slot group -(v+1).
 struct Combine {
-    DevBuf<int> seg, row0, ptr, idx;
+    DevBuf<int4> rows;
+    DevBuf<int> idx;
     DevBuf<ColSlots> groups;
     int64_t total = 0;          // list entries of all rows
     int64_t group_entries = 0;  // entries naming a column-slot group

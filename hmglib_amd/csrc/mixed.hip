@@ -700,18 +700,18 @@ lr_wg_kernel(const WgItem* __restrict__ items, const __bf16* __restrict__ Apan, 
 
 // Ys[i*32 + c] = sum of sorted row i's partials, in list order (deterministic)
 __global__ void __launch_bounds__(kThreads)
-combine_mx_kernel(const int* __restrict__ seg, const int* __restrict__ row0, const int* __restrict__ ptr,
-                  const int* __restrict__ idx, const float* __restrict__ P, float* __restrict__ Ys, int n1)
+combine_mx_kernel(const int4* __restrict__ rows, const int* __restrict__ idx, const float* __restrict__ P,
+                  float* __restrict__ Ys, int n1)
 {
     const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     const int i = (int)(t / kMxRhs), c = (int)(t % kMxRhs);
     if (i >= n1) return;
     // four partials loaded at a time, added in list order
-    const int sg = seg[i];
-    const float* __restrict__ Pi = P + (int64_t)(i - row0[sg]) * kMxRhs + c;
+    const int4 row = rows[i];
+    const float* __restrict__ Pi = P + (int64_t)row.z * kMxRhs + c;
     float s = 0.f;
-    int q = ptr[sg];
-    const int qe = ptr[sg + 1];
+    int q = row.x;
+    const int qe = row.y;
     for (; q + 4 <= qe; q += 4) {
         float v[4];
 #pragma unroll
@@ -956,7 +956,7 @@ hmg_status hmvp_mixed(Engine& eng, const Coords& c1, const Coords& c2, const Ker
         HMG_HIP(hipStreamWaitEvent(s, eng.ev_join, 0));
         eng.prof.begin(PROF_COMBINE, s);
         combine_mx_kernel<<<grid_for((int64_t)n1 * kMxRhs, kThreads), kThreads, 0, s>>>(
-            eng.comb_mx.seg.p, eng.comb_mx.row0.p, eng.comb_mx.ptr.p, eng.comb_mx.idx.p, eng.P32.p, eng.Ys32.p, n1);
+            eng.comb_mx.rows.p, eng.comb_mx.idx.p, eng.P32.p, eng.Ys32.p, n1);
         HMG_HIP(hipGetLastError());
         permute_out_kernel<<<grid_for(n1, kPermRows), kThreads, 0, s>>>(eng.Ys32.p, eng.inv1.p, Y, n1, c0, nr);
         HMG_HIP(hipGetLastError());

@@ -366,19 +366,18 @@ near_stored_kernel(const int4* __restrict__ items, int nitems, const int* __rest
 
 // y[order1[i]] = sum of row i's partials, in list order (a column-slot group
 // contributes its count slots of row i in order)
-__global__ void combine_kernel(const int* __restrict__ seg, const int* __restrict__ row0,
-                               const int* __restrict__ ptr, const int* __restrict__ idx,
+__global__ void combine_kernel(const int4* __restrict__ rows, const int* __restrict__ idx,
                                const ColSlots* __restrict__ groups, const double* __restrict__ P,
                                const uint64_t* __restrict__ order1, double* __restrict__ y, int n1)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n1) return;
-    const int sg = seg[i];
-    const double* __restrict__ Pi = P + (i - row0[sg]);
+    const int4 row = rows[i];
+    const double* __restrict__ Pi = P + row.z;
     double s = 0.0;
     // slots come before groups in a list; four loaded at a time, added in list order
-    int q = ptr[sg];
-    const int qe = ptr[sg + 1];
+    int q = row.x;
+    const int qe = row.y;
     for (; q + 4 <= qe && idx[q + 3] >= 0; q += 4) {
         double v[4];
 #pragma unroll
@@ -725,8 +724,8 @@ hmg_status hmvp_with(Engine& eng, const Coords& c1, const Coords& c2, const Kern
         HMG_HIP(hipStreamWaitEvent(s, eng.ev_join, 0));
         eng.prof.begin(PROF_COMBINE, s);
         const Combine& cb = dense_stored ? eng.comb_stored : eng.comb_fly;
-        combine_kernel<<<grid_for(n1, kThreads), kThreads, 0, s>>>(cb.seg.p, cb.row0.p, cb.ptr.p, cb.idx.p,
-                                                                   cb.groups.p, b.P, order1, yc, n1);
+        combine_kernel<<<grid_for(n1, kThreads), kThreads, 0, s>>>(cb.rows.p, cb.idx.p, cb.groups.p, b.P, order1,
+                                                                   yc, n1);
         HMG_HIP(hipGetLastError());
         eng.prof.end(PROF_COMBINE, s);
     }

@@ -345,16 +345,16 @@ near_multi_kernel(Coords c1, Coords c2, KernelParams kp, const int4* __restrict_
 // Ys[i*RB + c] = sum of sorted row i's partials P[v*RB + c], in list order
 template <int RB>
 __global__ void __launch_bounds__(kThreads)
-combine_multi_kernel(const int* __restrict__ seg, const int* __restrict__ row0, const int* __restrict__ ptr,
-                     const int* __restrict__ idx, const double* __restrict__ P, double* __restrict__ Ys, int n1)
+combine_multi_kernel(const int4* __restrict__ rows, const int* __restrict__ idx, const double* __restrict__ P,
+                     double* __restrict__ Ys, int n1)
 {
     const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     const int i = (int)(t / RB), c = (int)(t % RB);
     if (i >= n1) return;
-    const int sg = seg[i];
-    const double* __restrict__ Pi = P + (int64_t)(i - row0[sg]) * RB + c;
+    const int4 row = rows[i];
+    const double* __restrict__ Pi = P + (int64_t)row.z * RB + c;
     double s = 0.0;
-    for (int q = ptr[sg], qe = ptr[sg + 1]; q < qe; q++) s += Pi[(int64_t)idx[q] * RB];
+    for (int q = row.x; q < row.y; q++) s += Pi[(int64_t)idx[q] * RB];
     Ys[t] = s;
 }
 
@@ -438,7 +438,7 @@ hmg_status pass(Engine& eng, const Coords& c1, const Coords& c2, const KernelPar
     HMG_HIP(hipStreamWaitEvent(s, eng.ev_join, 0));
     eng.prof.begin(PROF_COMBINE, s);
     combine_multi_kernel<RB><<<grid_for((int64_t)n1 * RB, kThreads), kThreads, 0, s>>>(
-        eng.comb_stored.seg.p, eng.comb_stored.row0.p, eng.comb_stored.ptr.p, eng.comb_stored.idx.p, eng.P64.p, eng.Ys64.p, n1);
+        eng.comb_stored.rows.p, eng.comb_stored.idx.p, eng.P64.p, eng.Ys64.p, n1);
     HMG_HIP(hipGetLastError());
     permute_out_multi_kernel<RB><<<grid_for(n1, kRowTile), kThreads, 0, s>>>(eng.Ys64.p, eng.inv1.p, Y, n1, c0, nr);
     HMG_HIP(hipGetLastError());

@@ -162,10 +162,28 @@ __device__ __forceinline__ double kernel_value(const KernelParams& kp, double r2
 // second at the clock that such a stream of FMAs keeps).
 constexpr int kNearRows = 2 * kWave;
 // LDS reserved per near-field workgroup, which leaves wavefront slots to the low-rank
-// kernels beside it.  The matrix-free form needs its own (24 KB, six workgroups per compute
-// unit): 3D, N = 262144 7.7 ms with none, 8.1 with 32 KB, 10.0 with 64.  The stored one
-// streams: N = 50021 2.03 with none, 1.97 with 32, 2.11 with 64.
-constexpr int kFlyPad = 0, kStoredPad = 32 * 1024;
+// kernels beside it.  The stored form streams: N = 50021 2.03 ms with none, 1.97 with 32 KB,
+// 2.11 with 64.
+constexpr int kStoredPad = 32 * 1024;
+
+// The same for the matrix-free form, whose own LDS (24 KB) lets six workgroups onto a compute
+// unit; 32 KB more leave two.  Without a reservation the low-rank streams wait until the near
+// field has nearly ended; with it the two run side by side, the near field on fewer
+// wavefronts.  Products with none and with 32 KB, in ms (factor elements per evaluation):
+//   3D, leaf 256, rank 24: N = 131072 2.99, 3.17 (1.05); 180000 4.46, 4.73 (1.16);
+//     262144 7.53, 7.91 (0.97); 370000 11.98, 11.17 (1.27); 524288 19.1, 17.4 (1.20);
+//     1048576 42.9, 36.8 (2.08)
+//   3D, N = 262144: leaf 512 8.40, 8.58 (0.53); leaf 128 7.70, 7.19 (2.4)
+//   3D, N = 131072: two sets 3.20, 3.69 (0.55); rank 48 4.91, 4.45 (2.1)
+//   2D, leaf 64: N = 262144 2.30, 2.26 (18); 1048576 10.99, 10.92 (22);
+//     leaf 512: 65536 0.48, 0.39 (0.7); leaf 1024: 262144 1.80, 1.61 (0.6)
+// So none in three dimensions where the factors are not the longer part by some way, and none
+// on an engine of one stream, where nothing runs beside the near field.
+int fly_pad(const Engine& eng)
+{
+    if (eng.serialize || eng.stream == eng.stream2) return 0;
+    return eng.dim == 3 && 100 * eng.lr_elems < 118 * eng.near_evals ? 0 : 32 * 1024;
+}
 
 // lane i receives lane (i + 1) mod 64 of v (DPP wave_rol:1)
 __device__ __forceinline__ double lane_rotate_down(double v)
@@ -618,10 +636,10 @@ void launch_near_fly(bool reg, unsigned grid, hipStream_t s, const Coords& c1, c
 {
     double* Pnear = P + (int64_t)eng.n_lr_items * kTileRows;
     if (reg)
-        near_fly_kernel<KIND, DIM, true><<<grid, kThreads, eng.near_pad(kFlyPad), s>>>(
+        near_fly_kernel<KIND, DIM, true><<<grid, kThreads, eng.near_pad(fly_pad(eng)), s>>>(
             c1, c2, kp, eng.fly_items.p, eng.n_fly_items, eng.fly_refs.p, xs, Pnear, P);
     else
-        near_fly_kernel<KIND, DIM, false><<<grid, kThreads, eng.near_pad(kFlyPad), s>>>(
+        near_fly_kernel<KIND, DIM, false><<<grid, kThreads, eng.near_pad(fly_pad(eng)), s>>>(
             c1, c2, kp, eng.fly_items.p, eng.n_fly_items, eng.fly_refs.p, xs, Pnear, P);
 }
 

@@ -459,6 +459,7 @@ hmg_status aca_layout(Engine& eng, int k, int prec)
     int ntp = 0;
     eng.h_kb.assign(na, 0);
     eng.kmax = 0;
+    eng.lr_elems = 0;
     for (int a = 0; a < na; a++) {
         const int4 b = eng.h_blk[eng.ndense + a];
         const int m1 = b.y - b.x + 1, m2 = b.w - b.z + 1;
@@ -468,6 +469,7 @@ hmg_status aca_layout(Engine& eng, int k, int prec)
         if (kb < 0) kb = 0;
         eng.h_kb[a] = kb;
         eng.kmax = std::max(eng.kmax, kb);
+        eng.lr_elems += ((int64_t)m1 + m2) * kb;
     }
     // U and T in row-cluster (U) order
     eng.h_uoff.assign(na + 1, 0);

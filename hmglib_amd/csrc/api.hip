@@ -1433,8 +1433,8 @@ hmg_status hmg_set_option(struct h_matrix_data* data, int option, int64_t value)
         e->near_sym_enabled = value != 0;
         return HMG_OK;
     case HMG_OPT_NEAR_LDS_BYTES:
-        if (value < 0 || value > 128 * 1024) {
-            set_error("near-field LDS reservation must be in [0, 131072] bytes");
+        if (value < -1 || value > 128 * 1024) {
+            set_error("near-field LDS reservation must be in [0, 131072] bytes, or -1 (the kernel's choice)");
             return HMG_ERR_INVALID;
         }
         e->near_lds_pad = (int)value;

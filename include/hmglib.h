@@ -214,11 +214,10 @@ hmg_status hmg_get_schedule(const struct h_matrix_data* data, int64_t out[11]);
  * HMG_OPT_NEAR_SYMMETRIC [1]: when both sets are the same points, evaluate each
  *   transposed pair of DENSE blocks once (row and column sums); takes effect at
  *   the next setup_h_matrix.
- * HMG_OPT_NEAR_LDS_BYTES [the kernel's choice: for the matrix-free FP64 near field none
- *   or 32768, by the work beside it; 32768 for the stored one, 65536 for the
- *   mixed-precision one]: LDS reserved per near-field
- *   workgroup, which caps its occupancy so the low-rank streams keep wave slots
- *   beside it.
+ * HMG_OPT_NEAR_LDS_BYTES [-1]: LDS reserved per near-field workgroup, which caps its
+ *   occupancy so the low-rank streams keep wave slots beside it.  -1: the kernel's
+ *   choice (matrix-free FP64 near field none or 32768, by the work beside it; the
+ *   stored one 32768, the mixed-precision one 65536).
  * HMG_OPT_SERIALIZE [0]: run the near field on the main stream (no overlap).
  * HMG_OPT_PRECISION [HMG_PREC_FP64]: arithmetic of the next precompute_aca and
  *   of every product.  HMG_PREC_MIXED computes the ACA in FP64 exactly as

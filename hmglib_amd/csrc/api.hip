@@ -236,19 +236,34 @@ void large_free(void* p, size_t held)
 }
 
 namespace {
+// Kept buffers of one device: by size, and by age (the number of the put)
 struct IdleBlock {
     void* p;
     uint64_t age;
 };
 struct IdlePool {
-    std::mutex mu;
-    std::multimap<std::pair<int, size_t>, IdleBlock> blocks;  // by device and bytes
+    using Blocks = std::multimap<size_t, IdleBlock>;
+    Blocks blocks;
+    std::map<uint64_t, Blocks::iterator> ages;
     size_t bytes = 0;
+
+    void* take(Blocks::iterator it)
+    {
+        void* p = it->second.p;
+        bytes -= it->first;
+        ages.erase(it->second.age);
+        blocks.erase(it);
+        return p;
+    }
+};
+struct IdlePools {
+    std::mutex mu;
+    std::map<int, IdlePool> dev;
     uint64_t puts = 0;
 };
-IdlePool& idle_pool()
+IdlePools& idle_pools()
 {
-    static IdlePool* p = new IdlePool();  // never destroyed: see pin_pool
+    static IdlePools* p = new IdlePools();  // never destroyed: see pin_pool
     return *p;
 }
 // small ones are cheap in the device's pool
@@ -260,15 +275,14 @@ void* idle_take(size_t bytes, hipStream_t s, size_t* size)
 {
     int dev = 0;
     if (bytes < kIdleMin || hipStreamGetDevice(s, &dev) != hipSuccess) return nullptr;
-    IdlePool& pool = idle_pool();
-    std::lock_guard<std::mutex> lk(pool.mu);
-    const auto it = pool.blocks.lower_bound({dev, bytes});
-    if (it == pool.blocks.end() || it->first.first != dev || it->first.second > bytes + bytes / 4) return nullptr;
-    void* p = it->second.p;
-    *size = it->first.second;
-    pool.bytes -= *size;
-    pool.blocks.erase(it);
-    return p;
+    IdlePools& pools = idle_pools();
+    std::lock_guard<std::mutex> lk(pools.mu);
+    const auto at = pools.dev.find(dev);
+    if (at == pools.dev.end()) return nullptr;
+    const auto it = at->second.blocks.lower_bound(bytes);
+    if (it == at->second.blocks.end() || it->first > bytes + bytes / 4) return nullptr;
+    *size = it->first;
+    return at->second.take(it);
 }
 
 void idle_put(void* p, size_t size, hipStream_t s)
@@ -278,58 +292,60 @@ void idle_put(void* p, size_t size, hipStream_t s)
         (void)hipFreeAsync(p, s);
         return;
     }
-    void* out = p;
+    IdlePools& pools = idle_pools();
+    std::unique_lock<std::mutex> lk(pools.mu);
     try {
-        IdlePool& pool = idle_pool();
-        std::lock_guard<std::mutex> lk(pool.mu);
-        if (pool.bytes + size > kIdleBytes || pool.blocks.size() >= kIdleBlocks) {
-            // the oldest that makes room goes for it
-            auto old = pool.blocks.end();
-            for (auto it = pool.blocks.lower_bound({dev, 0}); it != pool.blocks.end() && it->first.first == dev; ++it)
-                if (pool.bytes - it->first.second + size <= kIdleBytes &&
-                    (old == pool.blocks.end() || it->second.age < old->second.age))
-                    old = it;
-            if (old != pool.blocks.end()) {
-                const IdleBlock b = old->second;
-                const size_t n = old->first.second;
-                pool.blocks.emplace(std::make_pair(dev, size), IdleBlock{p, pool.puts++});
-                pool.blocks.erase(old);
-                pool.bytes += size - n;
-                out = b.p;
-            }
-        } else {
-            pool.blocks.emplace(std::make_pair(dev, size), IdleBlock{p, pool.puts++});
-            pool.bytes += size;
-            out = nullptr;
+        IdlePool& pool = pools.dev[dev];
+        const uint64_t age = pools.puts++;
+        const auto it = pool.blocks.emplace(size, IdleBlock{p, age});
+        try {
+            pool.ages.emplace(age, it);
+        } catch (const std::bad_alloc&) {
+            pool.blocks.erase(it);
+            throw;
         }
+        pool.bytes += size;
     } catch (const std::bad_alloc&) {
+        lk.unlock();
+        (void)hipFreeAsync(p, s);
+        return;
     }
-    if (out) (void)hipFreeAsync(out, s);
+    // past the bounds the oldest go (frees outside the lock)
+    for (;;) {
+        const auto at = pools.dev.find(dev);  // (another thread may have trimmed meanwhile)
+        if (at == pools.dev.end()) return;
+        IdlePool& pool = at->second;
+        if (pool.bytes <= kIdleBytes && pool.blocks.size() <= kIdleBlocks) return;
+        void* old = pool.take(pool.ages.begin()->second);
+        lk.unlock();
+        (void)hipFreeAsync(old, s);
+        lk.lock();
+    }
 }
 
 void idle_trim(bool every)
 {
     int cur = 0;
     if (hipGetDevice(&cur) != hipSuccess) return;
-    std::multimap<std::pair<int, size_t>, IdleBlock> out;
+    std::map<int, IdlePool> out;
     {
-        IdlePool& pool = idle_pool();
-        std::lock_guard<std::mutex> lk(pool.mu);
-        for (auto it = pool.blocks.begin(); it != pool.blocks.end();) {
-            const auto at = it++;
-            if (!every && at->first.first != cur) continue;
-            pool.bytes -= at->first.second;
-            out.insert(pool.blocks.extract(at));
+        IdlePools& pools = idle_pools();
+        std::lock_guard<std::mutex> lk(pools.mu);
+        if (every) {
+            out.swap(pools.dev);
+        } else {
+            auto node = pools.dev.extract(cur);
+            if (node) out.insert(std::move(node));
         }
     }
-    for (auto it = out.begin(); it != out.end();) {
-        const int dev = it->first.first;
-        if (dev != cur) (void)hipSetDevice(dev);
-        for (; it != out.end() && it->first.first == dev; ++it) (void)hipFreeAsync(it->second.p, nullptr);
+    for (auto& d : out) {
+        if (d.second.blocks.empty()) continue;
+        if (d.first != cur) (void)hipSetDevice(d.first);
+        for (auto& b : d.second.blocks) (void)hipFreeAsync(b.second.p, nullptr);
         hipMemPool_t mp = nullptr;
-        if (hipDeviceSynchronize() == hipSuccess && hipDeviceGetDefaultMemPool(&mp, dev) == hipSuccess)
+        if (hipDeviceSynchronize() == hipSuccess && hipDeviceGetDefaultMemPool(&mp, d.first) == hipSuccess)
             (void)hipMemPoolTrimTo(mp, 0);
-        if (dev != cur) (void)hipSetDevice(cur);
+        if (d.first != cur) (void)hipSetDevice(cur);
     }
 }
 
@@ -658,6 +674,29 @@ void hmg_release_cached_memory(void)
     idle_trim(true);
     large_trim(true);
     pin_trim();
+}
+
+void hmg_cached_memory(int64_t out[6])
+{
+    if (!out) return;
+    for (int i = 0; i < 6; i++) out[i] = 0;
+    {
+        IdlePools& pools = idle_pools();
+        std::lock_guard<std::mutex> lk(pools.mu);
+        for (const auto& d : pools.dev) {
+            out[0] += (int64_t)d.second.bytes;
+            out[1] += (int64_t)d.second.blocks.size();
+        }
+    }
+    {
+        std::lock_guard<std::mutex> lk(g_large_mu);
+        for (const LargeBlock& b : g_large) out[2] += (int64_t)b.bytes;
+        out[3] = (int64_t)g_large.size();
+    }
+    PinPool& pins = pin_pool();
+    std::lock_guard<std::mutex> lk(pins.mu);
+    for (const PinBuf& b : pins.free) out[4] += (int64_t)b.bytes;
+    out[5] = (int64_t)pins.free.size();
 }
 
 // ------------------------------------------------------------------ init

@@ -98,7 +98,7 @@ void reclaim_device_memory();
 // the device's pool returns its free memory to the device whenever it exceeds the memory in
 // use (whatever its threshold), at 20 to 30 ms per GB both ways, which took 50 of the 75 ms
 // of destroying 24 clouds.  A buffer serves a request of at least four fifths of its size on its device.
-// At most kIdleBytes stay, the oldest go first; an allocation that fails and
+// At most kIdleBytes per device stay, the oldest go first; an allocation that fails and
 // hmg_release_cached_memory return them all.  Set on the thread that destroys
 // (IdleScope): releases go there.  (Streams are made anew: kept
 // ones, whose hardware queues then never change, made products 6 to 9 % slower.)

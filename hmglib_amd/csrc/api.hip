@@ -42,18 +42,20 @@ constexpr size_t kPinChunk = (size_t)4 << 20;
 // Pinned, device-mapped staging buffers (host and device addresses): each thread holds one
 // and hands it on when it ends.  A batched call starts its worker threads anew and each
 // grew a buffer of its own, request by request; hipHostMalloc and hipHostFree wait for the
-// device, and took 150 of 24 clouds' 190 ms.  At most kPinKept (64 MB) wait for another
-// thread; hmg_release_cached_memory returns those.
+// device, and took 150 of 24 clouds' 190 ms.  At most kPinKept (256 MB; as many as a server
+// has slots) wait for another thread.  An ending thread calls nothing of the runtime, which
+// may be gone with the process, so what is past the bound then waits apart, for the next
+// thread that takes a buffer or hmg_release_cached_memory to free it.
 struct PinBuf {
     void* host = nullptr;
     void* mapped = nullptr;
     size_t bytes = 0;
     int dev = 0;
 };
-constexpr size_t kPinKept = 16, kPinMin = (size_t)256 << 10;
+constexpr size_t kPinKept = 64, kPinMin = (size_t)256 << 10;
 struct PinPool {
     std::mutex mu;
-    std::vector<PinBuf> free;
+    std::vector<PinBuf> free, surplus;
 };
 PinPool& pin_pool()
 {
@@ -62,14 +64,15 @@ PinPool& pin_pool()
 }
 struct PinHolder {
     PinBuf b;
-    // No call of the runtime here, which may be gone when the process ends; a buffer past
-    // the bound stays with the process as the runtime's
     ~PinHolder()
     {
         if (!b.host) return;
         PinPool& p = pin_pool();
         std::lock_guard<std::mutex> lk(p.mu);
-        if (p.free.size() < kPinKept) p.free.push_back(b);
+        try {
+            (p.free.size() < kPinKept ? p.free : p.surplus).push_back(b);
+        } catch (const std::bad_alloc&) {  // stays with the process as the runtime's
+        }
     }
 };
 thread_local PinHolder t_pin;
@@ -79,7 +82,9 @@ void pin_trim()
     std::vector<PinBuf> out;
     {
         std::lock_guard<std::mutex> lk(pin_pool().mu);
-        out.swap(pin_pool().free);
+        out.swap(pin_pool().surplus);
+        out.insert(out.end(), pin_pool().free.begin(), pin_pool().free.end());
+        pin_pool().free.clear();
     }
     for (const PinBuf& b : out) (void)hipHostFree(b.host);
 }
@@ -91,13 +96,19 @@ hmg_status pinned(size_t bytes, void** host, void** dev)
         int d = 0;
         HMG_HIP(hipGetDevice(&d));
         PinPool& p = pin_pool();
-        std::lock_guard<std::mutex> lk(p.mu);
-        for (size_t i = p.free.size(); i-- > 0;) {
-            if (p.free[i].dev != d) continue;
-            b = p.free[i];
-            p.free.erase(p.free.begin() + (ptrdiff_t)i);
-            break;
+        std::vector<PinBuf> out;
+        {
+            std::lock_guard<std::mutex> lk(p.mu);
+            for (std::vector<PinBuf>* v : {&p.surplus, &p.free}) {
+                for (size_t i = v->size(); !b.host && i-- > 0;) {
+                    if ((*v)[i].dev != d) continue;
+                    b = (*v)[i];
+                    v->erase(v->begin() + (ptrdiff_t)i);
+                }
+            }
+            out.swap(p.surplus);
         }
+        for (const PinBuf& x : out) (void)hipHostFree(x.host);
     }
     if (b.bytes < bytes) {
         if (b.host) (void)hipHostFree(b.host);
@@ -695,8 +706,10 @@ void hmg_cached_memory(int64_t out[6])
     }
     PinPool& pins = pin_pool();
     std::lock_guard<std::mutex> lk(pins.mu);
-    for (const PinBuf& b : pins.free) out[4] += (int64_t)b.bytes;
-    out[5] = (int64_t)pins.free.size();
+    for (const std::vector<PinBuf>* v : {&pins.free, &pins.surplus}) {
+        for (const PinBuf& b : *v) out[4] += (int64_t)b.bytes;
+        out[5] += (int64_t)v->size();
+    }
 }
 
 // ------------------------------------------------------------------ init

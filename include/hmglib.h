@@ -331,12 +331,12 @@ const char* hmg_last_error(void);
  * same device (re-mapping device memory costs about 28 ms per GB on MI355X); this
  * returns them to the devices.  An allocation that fails returns them itself.
  * Also returned: up to 4 GiB per device of smaller buffers of destroyed H-matrices, kept for
- * later ones, and the pinned staging buffers (4 MiB each, 16 at most) of threads that
+ * later ones, and the pinned staging buffers (4 MiB each) of threads that
  * have ended. */
 void hmg_release_cached_memory(void);
 /* what that would return: out[0], out[1] = bytes and number of the smaller buffers kept,
  * out[2], out[3] = of the large ones, out[4], out[5] = of the staging buffers of ended
- * threads */
+ * threads (64 at most stay when another thread begins to copy) */
 void hmg_cached_memory(int64_t out[6]);
 /* sizeof / field offsets of the public structs, for FFI layout checks: which =
  * 0 h_matrix_data, 1 work_item, 2 point_set, 3 morton_code, 4 system_assembler,

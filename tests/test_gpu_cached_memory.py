@@ -65,3 +65,49 @@ def test_kept_buffers_stay_within_their_bounds(gpu):
     gpu.lib().hmg_release_cached_memory()
     assert _cached(gpu)["blocks"] == 0
     kern.free()
+
+
+def test_staging_buffers_of_ended_threads(gpu):
+    # more worker threads than buffers may wait: those past the bound are freed by the next
+    # thread that takes one, and none is lost
+    import threading
+
+    from hmglib_amd import hip
+    n_threads = 90
+    x = np.arange(64, dtype=np.float64)
+    kern = gpu.Kernel(O.K_EXPONENTIAL, 0.0, 0.1)
+    X = O.uniform(73, 2 * 600).reshape(2, 600)
+
+    def at_once(count):
+        hms = [gpu.HMatrix(X, X, 32, 1.0, 50, 64, 8) for _ in range(count)]
+        gate = threading.Barrier(count)
+
+        def work(hm):
+            gate.wait()
+            hm.setup()  # stages copies through the thread's buffer
+            gate.wait()
+
+        ts = [threading.Thread(target=work, args=(hm,)) for hm in hms]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        for hm in hms:
+            hm.destroy()
+
+    gpu.lib().hmg_release_cached_memory()
+    assert _cached(gpu)["pinned"] == 0
+    at_once(n_threads)
+    assert _cached(gpu)["pinned"] == n_threads
+    at_once(1)
+    assert _cached(gpu)["pinned"] <= 65
+    for _ in range(3):
+        at_once(n_threads)
+    at_once(1)
+    assert _cached(gpu)["pinned"] <= 65
+    gpu.lib().hmg_release_cached_memory()
+    assert _cached(gpu)["pinned"] == 0 and _cached(gpu)["pinned_bytes"] == 0
+    d = hip.DeviceArray(x)
+    np.testing.assert_array_equal(d.download(), x)
+    d.free()
+    kern.free()

@@ -164,6 +164,7 @@ hmg_status upload_bytes(void* dst, const void* src, size_t bytes, hipStream_t s)
         std::memcpy(pin, (const char*)src + off, n);
         const hmg_status ec = copy_bytes((char*)dst + off, pin_dev, n, s);
         const hipError_t es = hipStreamSynchronize(s);  // also on error: the buffer is reused
+        if (es == hipSuccess) idle_settle(s);
         if (ec != HMG_OK) {
             set_error("host-to-device copy launch failed");
             return ec;
@@ -182,6 +183,7 @@ hmg_status download_bytes(void* dst, const void* src, size_t bytes, hipStream_t 
         const size_t n = std::min(kPinChunk, bytes - off);
         const hmg_status ec = copy_bytes(pin_dev, (const char*)src + off, n, s);
         const hipError_t es = hipStreamSynchronize(s);
+        if (es == hipSuccess) idle_settle(s);
         if (ec != HMG_OK) {
             set_error("device-to-host copy launch failed");
             return ec;
@@ -331,6 +333,50 @@ void idle_put(void* p, size_t size, hipStream_t s)
         lk.unlock();
         (void)hipFreeAsync(old, s);
         lk.lock();
+    }
+}
+
+namespace {
+struct Deferred {
+    void* p;
+    size_t size;
+    hipStream_t s;
+};
+thread_local std::vector<Deferred> t_deferred;
+}  // namespace
+
+void idle_defer(void* p, size_t size, hipStream_t s)
+{
+    try {
+        t_deferred.push_back(Deferred{p, size, s});
+        if (g_alloc_stream) return;  // the scope's end at the latest
+        t_deferred.pop_back();
+    } catch (const std::bad_alloc&) {
+    }
+    (void)hipStreamSynchronize(s);
+    idle_put(p, size, s);
+}
+
+void idle_settle(hipStream_t s)
+{
+    if (t_deferred.empty()) return;
+    size_t left = 0;
+    for (size_t i = 0; i < t_deferred.size(); i++) {
+        const Deferred d = t_deferred[i];
+        if (d.s == s)
+            idle_put(d.p, d.size, d.s);
+        else
+            t_deferred[left++] = d;
+    }
+    t_deferred.resize(left);
+}
+
+void idle_settle_all()
+{
+    while (!t_deferred.empty()) {
+        const hipStream_t s = t_deferred.back().s;
+        (void)hipStreamSynchronize(s);
+        idle_settle(s);
     }
 }
 
@@ -1615,13 +1661,14 @@ hmg_status hmg_destroy_h_matrix_data(struct h_matrix_data* data)
     if (!e) return HMG_OK;
     // finish the engine's work, then return every buffer on its own stream
     // (stream-ordered frees do not wait for other H-matrices' kernels).  With a
-    // caller-owned stream the caller has finished this H-matrix's work already.
+    // caller-owned stream the caller has finished this H-matrix's work already, also
+    // after a call that failed.
     if (e->own_streams) {
         (void)hipStreamSynchronize(e->stream2);
         (void)hipStreamSynchronize(e->stream);
     }
     hipStream_t s = e->stream;
-    IdleScope idle(e->own_streams);
+    IdleScope idle(true);
     {
         AllocScope scope(s);
         release_build(*e, data);

@@ -70,10 +70,15 @@ struct Coords {
 // concurrently wait for the kernels of all others whenever one frees a buffer.
 // Outside a scope DevBuf uses plain hipMalloc / hipFree.
 extern thread_local hipStream_t g_alloc_stream;
+void idle_settle_all();
 struct AllocScope {
     hipStream_t prev;
     explicit AllocScope(hipStream_t s) : prev(g_alloc_stream) { g_alloc_stream = s; }
-    ~AllocScope() { g_alloc_stream = prev; }
+    ~AllocScope()
+    {
+        idle_settle_all();
+        g_alloc_stream = prev;
+    }
     AllocScope(const AllocScope&) = delete;
     AllocScope& operator=(const AllocScope&) = delete;
 };
@@ -94,7 +99,8 @@ void large_trim(bool every);
 // is idle, the stream-ordered pool's free memory of the current device
 void reclaim_device_memory();
 
-// Buffers of a destroyed H-matrix, whose streams were waited for, are kept for later ones:
+// Buffers of a destroyed H-matrix and a build's scratch, whose streams were waited for, are
+// kept for later ones:
 // the device's pool returns its free memory to the device whenever it exceeds the memory in
 // use (whatever its threshold), at 20 to 30 ms per GB both ways, which took 50 of the 75 ms
 // of destroying 24 clouds.  A buffer serves a request of at least four fifths of its size on its device.
@@ -119,8 +125,17 @@ inline size_t idle_size(size_t bytes)
     while (bytes / q >= 32) q *= 2;
     return bytes < 4096 ? bytes : (bytes + q - 1) / q * q;
 }
+// A kept buffer may have been allocated on any stream, and the device's pool takes that
+// stream (and a later one with its handle) for one that may have the buffer back at once,
+// whatever still uses it on the stream that frees it (seen on MI355X, ROCm 7.2).  So it is
+// never freed in stream order: released while work may still use it, it waits on the
+// releasing thread until its stream has been waited for, and is kept again then.
 // a kept buffer for `bytes` on the stream's device (its size in *size), or nullptr
 void* idle_take(size_t bytes, hipStream_t s, size_t* size);
+// releases a buffer that idle_take gave, behind the work queued on s
+void idle_defer(void* p, size_t size, hipStream_t s);
+// s has been waited for: the buffers that this thread deferred behind it are kept
+void idle_settle(hipStream_t s);
 // keeps p, which no work uses any more; `s`, a stream of its device, frees what has to go for it
 void idle_put(void* p, size_t size, hipStream_t s);
 // returns the kept buffers of the current device (all devices: every = true)
@@ -133,10 +148,11 @@ struct DevBuf {
     hipStream_t s = nullptr;  // allocation stream (nullptr: hipMalloc)
     size_t held = 0;          // bytes of a large buffer (from the large-buffer cache)
     size_t size = 0;          // bytes of a stream-ordered buffer
+    bool kept = false;        // it was a kept buffer (idle_take)
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n), s(o.s), held(o.held), size(o.size)
+    DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n), s(o.s), held(o.held), size(o.size), kept(o.kept)
     {
         o.p = nullptr;
         o.n = 0;
@@ -152,6 +168,7 @@ struct DevBuf {
             s = o.s;
             held = o.held;
             size = o.size;
+            kept = o.kept;
             o.p = nullptr;
             o.n = 0;
             o.s = nullptr;
@@ -175,6 +192,7 @@ struct DevBuf {
             st = g_alloc_stream;
             size = st ? idle_size(bytes) : bytes;
             p = st ? (T*)idle_take(bytes, st, &size) : nullptr;
+            kept = p != nullptr;
             e = p ? hipSuccess : st ? hipMallocAsync((void**)&p, size, st) : hipMalloc(&p, bytes);
             if (e != hipSuccess) {
                 // cached large buffers or the pool may hold the memory: return it and retry
@@ -202,6 +220,8 @@ struct DevBuf {
                 large_free(p, held);
             else if (s && g_alloc_idle)
                 idle_put(p, size, s);
+            else if (s && kept)
+                idle_defer(p, size, s);
             else if (s)
                 (void)hipFreeAsync(p, s);
             else
@@ -211,6 +231,7 @@ struct DevBuf {
         n = 0;
         s = nullptr;
         held = 0;
+        kept = false;
     }
 };
 

@@ -120,8 +120,11 @@ void finish(hmg_server* s, Request* r, int status, double t_end)
 // kernel descriptor goes back to the server's free list
 void destroy_matrix(hmg_server* s, Matrix* m)
 {
-    m->Xb.release();
-    m->Yb.release();
+    {
+        IdleScope idle(true);  // every pass waited for its stream
+        m->Xb.release();
+        m->Yb.release();
+    }
     if (m->inited) (void)hmg_destroy_h_matrix_data(&m->data);
     m->inited = false;
     if (m->kern) {
@@ -257,6 +260,7 @@ hmg_status run_build(hmg_server* s, Matrix* m, Request* r, hipStream_t slot, std
     }
     int64_t mem[2] = {0, 0};
     if (st == HMG_OK) st = hmg_memory(&d, mem);
+    if (st != HMG_OK) (void)hipStreamSynchronize(slot);
     lk.lock();
     if (st != HMG_OK) return st;
     // admission: the tree is built; the factors and product buffers must fit
@@ -284,6 +288,8 @@ hmg_status run_build(hmg_server* s, Matrix* m, Request* r, hipStream_t slot, std
     m->bytes = need;
     lk.unlock();
     st = hmg_precompute_aca(&d);
+    // after a failure its launches may still run, and the buffers go to other H-matrices next
+    if (st != HMG_OK) (void)hipStreamSynchronize(slot);
     lk.lock();
     return st;
 }
@@ -327,6 +333,7 @@ hmg_status run_pass(hmg_server* s, Matrix* m, std::vector<Request*>& batch, int 
         }
         if (st == HMG_OK && hipStreamSynchronize(e->stream) != hipSuccess) st = HMG_ERR_HIP;
     }
+    if (st != HMG_OK) (void)hipStreamSynchronize(e->stream);
     lk.lock();
     return st;
 }

@@ -11,7 +11,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 # state: the states that captured products are compared with differ between successive H-matrices
 # options: the near field's LDS reservation is set and given back
-@pytest.mark.parametrize("name", ["state", "options"])
+# kept: a kept buffer is not freed or handed on before its stream was waited for
+@pytest.mark.parametrize("name", ["state", "options", "kept"])
 def test_host_program(tmp_path, name):
     exe = str(tmp_path / name)
     subprocess.run([build.hipcc()] + build.FLAGS +

@@ -704,8 +704,9 @@ constexpr int kAcaRounds = 64;
 // long searches again.
 constexpr int kRegTries = 64, kWideTries = 32, kWideRetries = 8;
 constexpr int kAcaBlind = 4;  // rounds between two looks at the queues
-// bound of a wide class' slabs together
-constexpr int64_t kSlabBytes = (int64_t)3 << 30;
+// Bounds of a wide class' slabs together: of an engine with two streams, and of one with a
+// single stream, which shares the chip with other such engines
+constexpr int64_t kSlabBytes = (int64_t)3 << 30, kSlabShared = (int64_t)256 << 20;
 
 static int aca_class(const Engine& eng, const KernelParams& kp, int a)
 {
@@ -806,13 +807,36 @@ static hmg_status search_launch(const AcaArgs& g, int maxm1, hipStream_t s)
     }
 }
 
-// Scratch of the register form's launches (grown as needed)
+// Scratch of the register form's launches (grown as needed).  An engine with one stream, a
+// server's slot, takes it from the scratch that is kept per stream: allocated by every build
+// it made the device's pool grow and shrink, which then held all slots up by turns.
 struct AcaWork {
-    DevBuf<int> ints;  // [counters][two queues][row][found]
-    DevBuf<double> fro2, slabs[kWide];
-    int cus = 0;  // compute units
-    hmg_status init()
+    int* ints = nullptr;  // [counters][two queues][row][found]
+    double *fro2 = nullptr, *slabs[kWide] = {nullptr, nullptr};
+    DevBuf<int> own_ints;
+    DevBuf<double> own_fro2, own_slabs[kWide];
+    hipStream_t s = nullptr, s2 = nullptr;
+    bool running = false;
+    ~AcaWork()
     {
+        if (!running) return;  // a failed build: its launches may still use the buffers
+        (void)hipStreamSynchronize(s2);
+        (void)hipStreamSynchronize(s);
+    }
+    bool shared() const { return s == s2; }
+    template <class T>
+    hmg_status get(DevBuf<T>& own, int slot, size_t n, T** p)
+    {
+        if (shared()) return scratch_of_stream(s, kAcaScratch + slot, n * sizeof(T), (void**)p);
+        HMG_TRY(own.alloc(n));
+        *p = own.p;
+        return HMG_OK;
+    }
+    int cus = 0;  // compute units
+    hmg_status init(const Engine& eng)
+    {
+        s = eng.stream;
+        s2 = eng.stream2;
         int dev = 0;
         HMG_HIP(hipGetDevice(&dev));
         HMG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -820,7 +844,27 @@ struct AcaWork {
     }
     // so many teams leave part of the chip idle (two per compute unit fill it)
     int few() const { return 2 * cus; }
+    // slabs of a wide class: one per workgroup that the chip holds, as far as they fit
+    int slab_count(const AcaCounts& cnt, int i) const
+    {
+        const int n = cnt.n[kRegClass + i];
+        if (n == 0) return 0;
+        const int64_t fit = (shared() ? kSlabShared : kSlabBytes) / (std::max<int64_t>(cnt.slab[i], 1) * 8);
+        return (int)std::min<int64_t>(std::min(n, std::max(cus, 1) * (i == 0 ? 1 : 3)), std::max<int64_t>(fit, 1));
+    }
 };
+
+int64_t aca_work_bytes(const Engine& eng, const KernelParams& kp)
+{
+    AcaWork work;
+    if (work.init(eng) != HMG_OK) return 0;
+    std::vector<int> all(eng.naca), list;
+    for (int a = 0; a < eng.naca; a++) all[a] = a;
+    const AcaCounts cnt = aca_order(eng, kp, all, work.few(), list);
+    int64_t bytes = (int64_t)eng.naca * 24;  // queues, rows, sums
+    for (int i = 0; i < kWide; i++) bytes += 8 * cnt.slab[i] * work.slab_count(cnt, i);
+    return work.shared() ? bytes + bytes / 4 : bytes;  // (scratch of a stream grows by more than asked)
+}
 
 // The blocks of list[] (aca_order), factor offsets uoff / voff (leading dims eng.ldu /
 // eng.ldv) into U / V or block pointers ublk / vblk.  The classes are dealt to the
@@ -847,21 +891,20 @@ static hmg_status aca_launch(Engine& eng, const Coords& c1, const Coords& c2, co
     int nslabs[kWide] = {0};
     if (nreg > 0) {
         const int na = eng.naca;
-        HMG_TRY(work.ints.alloc((size_t)kCounters + 2 * (size_t)nreg + 2 * (size_t)na));
-        HMG_TRY(work.fro2.alloc((size_t)na));
+        HMG_TRY(work.get(work.own_ints, 0, (size_t)kCounters + 2 * (size_t)nreg + 2 * (size_t)na, &work.ints));
+        HMG_TRY(work.get(work.own_fro2, 1, (size_t)na, &work.fro2));
         for (int i = 0; i < kWide; i++) {
             if (cnt.n[kRegClass + i] == 0) continue;
-            const int64_t fit = std::max<int64_t>(kSlabBytes / (std::max<int64_t>(cnt.slab[i], 1) * 8), 1);
-            nslabs[i] = (int)std::min<int64_t>(std::min(cnt.n[kRegClass + i], std::max(work.cus, 1) * (i == 0 ? 1 : 3)),
-                                               fit);
+            nslabs[i] = work.slab_count(cnt, i);
             // short of memory: fewer slabs; none at all: the memory form
-            while (nslabs[i] > 0 && work.slabs[i].alloc((size_t)(cnt.slab[i] * nslabs[i])) != HMG_OK) {
+            while (nslabs[i] > 0 && work.get(work.own_slabs[i], 2 + i, (size_t)(cnt.slab[i] * nslabs[i]),
+                                             &work.slabs[i]) != HMG_OK) {
                 (void)hipGetLastError();
                 nslabs[i] /= 2;
             }
         }
     }
-    int* const counters = work.ints.p;
+    int* const counters = work.ints;
     AcaArgs g{};
     g.c1 = c1;
     g.c2 = c2;
@@ -886,7 +929,7 @@ static hmg_status aca_launch(Engine& eng, const Coords& c1, const Coords& c2, co
     if (nreg > 0) {
         g.row = counters + kCounters + 2 * (size_t)nreg;
         g.found = g.row + eng.naca;
-        g.fro2 = work.fro2.p;
+        g.fro2 = work.fro2;
         HMG_HIP(hipMemsetAsync(counters, 0, kCounters * sizeof(int), s));
     }
     const bool two = s2 != s;
@@ -904,6 +947,7 @@ static hmg_status aca_launch(Engine& eng, const Coords& c1, const Coords& c2, co
         }
         return HMG_OK;
     };
+    work.running = true;
     HMG_TRY(fork());
     if (cnt.n[0] > 0) {
         if (tol.mode != 0) {
@@ -962,7 +1006,7 @@ static hmg_status aca_launch(Engine& eng, const Coords& c1, const Coords& c2, co
                 g.suspend = g.scan && round < kAcaRounds ? 1 : 0;
                 g.tries = !wide ? kRegTries : round == 0 ? kWideTries : kWideRetries;
                 if (wide) {
-                    g.slabs = work.slabs[c - kRegClass].p;
+                    g.slabs = work.slabs[c - kRegClass];
                     g.slab = cnt.slab[c - kRegClass];
                     g.nslabs = nslabs[c - kRegClass];
                 }
@@ -972,17 +1016,19 @@ static hmg_status aca_launch(Engine& eng, const Coords& c1, const Coords& c2, co
         }
         round += rounds;
         HMG_TRY(join());
-        if (!g.scan) return HMG_OK;
+        if (!g.scan) break;
         // the blocks queued by the look's last round are the first row of the next one
         HMG_TRY(download_bytes(n, counters + rounds * kRow, sizeof(int) * kClasses, s));
         bool any = false;
         for (int c = kRegClass; c < kClasses; c++) any = any || n[c] > 0;
-        if (!any) return HMG_OK;
+        if (!any) break;
         HMG_HIP(hipMemsetAsync(counters, 0, kCounters * sizeof(int), s));
         HMG_TRY(upload_bytes(counters, n, sizeof(int) * kClasses, s));
         HMG_TRY(fork());
     }
-    return join();
+    if (nreg == 0) HMG_TRY(join());
+    work.running = false;
+    return HMG_OK;
 }
 
 hmg_status aca_build(Engine& eng, const Coords& c1, const Coords& c2, const KernelParams& kp, int k,
@@ -996,7 +1042,7 @@ hmg_status aca_build(Engine& eng, const Coords& c1, const Coords& c2, const Kern
     for (int a = 0; a < na; a++) all[a] = a;
     eng.h_aca_list.clear();
     AcaWork work;
-    HMG_TRY(work.init());
+    HMG_TRY(work.init(eng));
     const AcaCounts cnt = aca_order(eng, kp, all, work.few(), eng.h_aca_list);
     HMG_TRY(eng.aca_list.alloc(na));
     HMG_TRY(upload_bytes(eng.aca_list.p, eng.h_aca_list.data(), sizeof(int) * na, s));
@@ -1142,7 +1188,7 @@ hmg_status aca_build_mixed(Engine& eng, const Coords& c1, const Coords& c2, cons
     list.reserve(na);
     std::vector<int> bptr(nb + 1, 0);
     AcaWork work;
-    HMG_TRY(work.init());
+    HMG_TRY(work.init(eng));
     std::vector<AcaCounts> cnt(nb);
     for (int q = 0; q < nb; q++) {
         bptr[q] = (int)list.size();

@@ -587,6 +587,12 @@ Engine* engine_of(const h_matrix_data* d);
 // The primitives keep grow-only scratch buffers per (stream, slot); an engine
 // releases the scratch of its streams when it is destroyed.
 void release_scratch(hipStream_t s);
+// scratch of at least `bytes` that stays with the stream until release_scratch; one buffer
+// per slot, grown in stream order (slots up to kAcaScratch - 1 are the primitives' own)
+constexpr int kAcaScratch = 1000;
+int64_t scratch_bytes(hipStream_t s, int from);
+void release_scratch(hipStream_t s, int from);
+hmg_status scratch_of_stream(hipStream_t s, int slot, size_t bytes, void** out);
 // exclusive or inclusive scan of int32, n elements, in -> out (may alias);
 // optional device pointer `total` receives the sum.
 hmg_status scan_i32(const int* in, int* out, int64_t n, bool inclusive, int* total,
@@ -697,6 +703,10 @@ hmg_status aca_build(Engine& eng, const Coords& c1, const Coords& c2, const Kern
 hmg_status aca_build_mixed(Engine& eng, const Coords& c1, const Coords& c2, const KernelParams& kp,
                            int tie_last, __bf16* Up, __bf16* Vp);
 // FP64 scratch elements aca_build_mixed uses for the current layout
+// hmg_memory for a kernel of that kind
+hmg_status memory_of(const h_matrix_data* data, int kind, int64_t out[2]);
+// bytes of scratch that the ACA of every block takes beside the factors
+int64_t aca_work_bytes(const Engine& eng, const KernelParams& kp);
 int64_t aca_mixed_scratch(const Engine& eng);
 // BF16 hi + lo panels (Up / Vp) of ACA blocks list[0 .. n) of eng from FP64
 // factors in a scratch: U_b column-major (ld m1) at S + suoff[a], V_b row-major (ld

@@ -301,19 +301,29 @@ differ_kernel(const uint64_t* __restrict__ a, const uint64_t* __restrict__ b, in
 
 }  // namespace
 
-void release_scratch(hipStream_t s)
+hmg_status scratch_of_stream(hipStream_t s, int slot, size_t bytes, void** out) { return scratch(s, slot, bytes, out); }
+
+int64_t scratch_bytes(hipStream_t s, int from)
 {
     ScratchCache& c = scratch_cache();
     std::lock_guard<std::mutex> g(c.mu);
-    for (auto it = c.bufs.begin(); it != c.bufs.end();) {
-        if (it->first.first == s) {
-            it->second.release();
-            it = c.bufs.erase(it);
-        } else {
-            ++it;
-        }
+    int64_t t = 0;
+    for (auto it = c.bufs.lower_bound({s, from}); it != c.bufs.end() && it->first.first == s; ++it)
+        t += (int64_t)it->second.n;
+    return t;
+}
+
+void release_scratch(hipStream_t s, int from)
+{
+    ScratchCache& c = scratch_cache();
+    std::lock_guard<std::mutex> g(c.mu);
+    for (auto it = c.bufs.lower_bound({s, from}); it != c.bufs.end() && it->first.first == s;) {
+        it->second.release();
+        it = c.bufs.erase(it);
     }
 }
+
+void release_scratch(hipStream_t s) { release_scratch(s, 0); }
 
 hmg_status scan_i32(const int* in, int* out, int64_t n, bool inclusive, int* total, hipStream_t s)
 {

@@ -1422,7 +1422,7 @@ template <class T>
 int64_t bytes_of(const DevBuf<T>& b)
 {
     if (!b.p) return 0;
-    return b.held ? (int64_t)b.held : (int64_t)b.n * (int64_t)sizeof(T);
+    return b.held ? (int64_t)b.held : (int64_t)std::max(b.size, b.n * sizeof(T));
 }
 
 int64_t engine_bytes(const Engine& e)
@@ -1448,7 +1448,11 @@ int64_t engine_bytes(const Engine& e)
 }  // namespace
 }  // extern "C++"
 
-hmg_status hmg_memory(const struct h_matrix_data* data, int64_t out[2])
+}  // extern "C"
+
+namespace hmg {
+
+hmg_status memory_of(const h_matrix_data* data, int kind, int64_t out[2])
 {
     Engine* e = engine_of(data);
     if (!e || !out) {
@@ -1473,6 +1477,10 @@ hmg_status hmg_memory(const struct h_matrix_data* data, int64_t out[2])
         // mixed: BF16 hi + lo panels (4 bytes per element, padded to whole MFMA
         // tiles) plus the FP64 scratch of the ACA batches
         add += mixed ? (int64_t)(elems * 4.0 * 1.25) + 8 * aca_mixed_scratch(*e) : (int64_t)(elems * 8.0);
+        KernelParams kp{};
+        kp.kind = kind;
+        kp.dim = e->dim;
+        add += aca_work_bytes(*e, kp);
     }
     if (mixed && e->layout_prec != HMG_PREC_MIXED) {
         const int64_t n1 = e->n[0], n2 = e->n[1];
@@ -1516,6 +1524,16 @@ hmg_status hmg_memory(const struct h_matrix_data* data, int64_t out[2])
     }
     out[1] = add + add / 10 + (64 << 20);
     return HMG_OK;
+}
+
+}  // namespace hmg
+
+extern "C" {
+
+// (any kernel may follow: one whose ACA takes the most scratch)
+hmg_status hmg_memory(const struct h_matrix_data* data, int64_t out[2])
+{
+    return memory_of(data, HMG_KERNEL_GAUSSIAN, out);
 }
 
 hmg_status hmg_set_option(struct h_matrix_data* data, int option, int64_t value)

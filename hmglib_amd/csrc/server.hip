@@ -259,21 +259,33 @@ hmg_status run_build(hmg_server* s, Matrix* m, Request* r, hipStream_t slot, std
         d.assem = m->kern;
     }
     int64_t mem[2] = {0, 0};
-    if (st == HMG_OK) st = hmg_memory(&d, mem);
+    if (st == HMG_OK) st = memory_of(&d, b.kernel_kind, mem);
     if (st != HMG_OK) (void)hipStreamSynchronize(slot);
     lk.lock();
     if (st != HMG_OK) return st;
-    // admission: the tree is built; the factors and product buffers must fit
+    // admission: the tree is built; the factors and product buffers must fit beside the
+    // scratch that the other slots keep for their next ACA (this one's is part of the need)
     const int64_t need = mem[0] + mem[1];
     for (;;) {
-        std::vector<std::unique_ptr<Matrix>> victims = make_room(s, need);
+        int64_t held = 0;
+        for (hipStream_t st2 : s->slot_streams)
+            if (st2 != slot) held += scratch_bytes(st2, kAcaScratch);
+        // rather than evict or fail for it, it is given back: where this is the only job that
+        // does not wait, no ACA runs on any slot, and none begins while the lock is held
+        if (held > 0 && s->used + need + held > s->cfg.hbm_budget_bytes && s->running - s->waiting <= 1) {
+            IdleScope idle(true);
+            for (hipStream_t st2 : s->slot_streams)
+                if (st2 != slot) release_scratch(st2, kAcaScratch);
+            held = 0;
+        }
+        std::vector<std::unique_ptr<Matrix>> victims = make_room(s, need + held);
         if (!victims.empty()) {
             lk.unlock();
             for (auto& v : victims) destroy_matrix(s, v.get());
             victims.clear();
             lk.lock();
         }
-        if (s->used + need <= s->cfg.hbm_budget_bytes) break;
+        if (s->used + need + held <= s->cfg.hbm_budget_bytes) break;
         // fail unless some other job that is not itself waiting can still free memory
         if (s->running - s->waiting <= 1) {
             set_error("H-matrix needs " + std::to_string(need) + " bytes; the budget of " +

@@ -14,6 +14,7 @@
 //   accumulated as fma(-s, w, val) in l order (nvcc's contraction of :955/:1143).
 // The 2-norm is a wavefront FP64 reduction; the argmax a (|v|, index, v) butterfly.
 #include <algorithm>
+#include <cmath>
 
 #include "aca_reg.h"
 #include "hmg_internal.h"
@@ -703,6 +704,13 @@ constexpr int kAcaRounds = 64;
 // trip; a wide one takes up to thirty per row, and the blocks suspended once mostly have
 // long searches again.
 constexpr int kRegTries = 64, kWideTries = 32, kWideRetries = 8;
+// Where a class' teams leave part of the chip idle, a search counts by its length and not by
+// the team that it holds up: blocks of up to so many entries are not suspended there.  The
+// ACA of N = 8192, without and with: 2D uniform 2.9 and 6.3 ms, 2D clouds 4.4 and 7.4, 3D
+// clouds 5.1 and 6.3 (the memory form took 4.5, 7.6 and 5.6); a block of 4096 rows and columns
+// is better suspended (N = 16384, 2D clouds 16 and 27), and so are teams of 16, whose rows
+// cost most, where such blocks make rounds in any case (N = 16384, 2D uniform 15.5 and 17.4).
+constexpr int64_t kSearchAlone = (int64_t)1 << 22;
 constexpr int kAcaBlind = 4;  // rounds between two looks at the queues
 // Bounds of a wide class' slabs together: of an engine with two streams, and of one with a
 // single stream, which shares the chip with other such engines
@@ -731,7 +739,7 @@ struct AcaCounts {
     int n[kClasses] = {0};
     int kmax[kClasses] = {0};
     int m1max[kClasses] = {0};
-    double work[kClasses] = {0.0};  // rows and columns times rank
+    int64_t area[kClasses] = {0};   // largest block's entries
     int64_t slab[kWide] = {0};
 };
 
@@ -763,8 +771,8 @@ static AcaCounts aca_order(const Engine& eng, const KernelParams& kp, const std:
     for (size_t q = 0; q < members.size(); q++) {
         const int a = members[q], i = cls[q];
         const int4 b = eng.h_blk[eng.ndense + a];
-        c.work[i] += ((double)(b.y - b.x + 1) + (b.w - b.z + 1)) * eng.h_kb[a];
         c.m1max[i] = std::max(c.m1max[i], b.y - b.x + 1);
+        c.area[i] = std::max(c.area[i], (int64_t)(b.y - b.x + 1) * (b.w - b.z + 1));
         if (i >= kRegClass && i < kRegClass + kWide)
             c.slab[i - kRegClass] = std::max(c.slab[i - kRegClass], (int64_t)(b.w - b.z + 1) * eng.h_kb[a]);
     }
@@ -866,10 +874,23 @@ int64_t aca_work_bytes(const Engine& eng, const KernelParams& kp)
     return work.shared() ? bytes + bytes / 4 : bytes;  // (scratch of a stream grows by more than asked)
 }
 
+// About how long n teams of class c run (us): a rank step's latency by team and block size
+// (a team of 16 wavefronts 24 us, of one 6; a wide one 50 at 4096 columns), the ranks, and
+// the teams that a compute unit runs one after another.  Dealt by rows, columns and ranks
+// alone, small builds left one stream idle for a third of the time (N = 4096, 2D clouds, ACA
+// 3.2 ms).
+static double class_time(const AcaCounts& cnt, int c, int n, int cus)
+{
+    const int nw = kRegWaves[c - kRegClass];
+    const bool wide = c < kRegClass + kWide;
+    const double step = wide ? 10.0 + std::sqrt((double)cnt.area[c]) / (64.0 * nw) * 5.0 : 5.0 + 1.2 * nw;
+    return std::max(1.0, (double)n * nw / (12.0 * std::max(cus, 1))) * cnt.kmax[c] * step;
+}
+
 // The blocks of list[] (aca_order), factor offsets uoff / voff (leading dims eng.ldu /
 // eng.ldv) into U / V or block pointers ublk / vblk.  The classes are dealt to the
-// engine's two streams, the one with less work so far first, so that one's last workgroups
-// run beside the next; both are joined back.  Rounds: blocks that suspended themselves are searched and resumed until
+// engine's two streams, the longest first, to the one with less to do so far, so that one's
+// last workgroups run beside the next; both are joined back.  Rounds: blocks that suspended themselves are searched and resumed until
 // none is left (each round raises the rank or the row of every one of them); the host
 // looks at the queues once per kAcaBlind rounds, the launches in between end at once
 // where their queue is empty.
@@ -983,17 +1004,24 @@ static hmg_status aca_launch(Engine& eng, const Coords& c1, const Coords& c2, co
         HMG_HIP(hipGetLastError());
         n[c] = 0;
     }
+    bool rounds_anyway = false;
+    for (int c = kRegClass; c < kClasses; c++) rounds_anyway = rounds_anyway || cnt.area[c] > kSearchAlone;
     for (int round = 0; nreg > 0;) {
         // one look: the blocks themselves, or kAcaBlind rounds of the suspended ones
         const int rounds = round == 0 ? 1 : kAcaBlind;
         double load[2] = {0.0, 0.0};
-        for (int c = kRegClass; c < kClasses; c++) {
-            if (n[c] == 0) continue;
+        std::vector<std::pair<double, int>> deal;
+        for (int c = kRegClass; c < kClasses; c++)
+            if (n[c] > 0) deal.emplace_back(class_time(cnt, c, n[c], work.cus), c);
+        std::sort(deal.begin(), deal.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+        for (const auto& [time, c] : deal) {
             const bool wide = c < kRegClass + kWide;
             const int to = load[0] <= load[1] ? 0 : 1;
-            load[to] += cnt.work[c] * n[c] / cnt.n[c];
+            load[to] += time;
             hipStream_t sc = to == 0 ? s : s2;
             const int at = first[c] - first[kRegClass];
+            const bool alone = cnt.n[c] <= work.few() && cnt.area[c] <= kSearchAlone &&
+                               !(rounds_anyway && kRegWaves[c - kRegClass] == 16);
             for (int q = 0; q < rounds; q++) {
                 const int parity = (round + q) & 1;
                 g.list = round == 0 ? list + first[c] : counters + kCounters + (size_t)parity * nreg + at;
@@ -1003,7 +1031,7 @@ static hmg_status aca_launch(Engine& eng, const Coords& c1, const Coords& c2, co
                 g.queued = counters + (q + 1) * kRow + c;
                 g.next = counters + q * kRow + 16 + (c - kRegClass);
                 g.resume = round > 0 ? 1 : 0;
-                g.suspend = g.scan && round < kAcaRounds ? 1 : 0;
+                g.suspend = g.scan && round < kAcaRounds && !alone ? 1 : 0;
                 g.tries = !wide ? kRegTries : round == 0 ? kWideTries : kWideRetries;
                 if (wide) {
                     g.slabs = work.slabs[c - kRegClass];

@@ -1151,8 +1151,8 @@ hmg_status reg_launch_nw(const AcaArgs& g, int nw, bool wide, int kmax, hipStrea
     const unsigned n = (unsigned)g.nlist;
     if (wide) {
         const unsigned m = (unsigned)std::min(g.nlist, g.nslabs);
-        // few resumed blocks: eight wavefronts halve a rank step's latency
-        if (nw == 4 && !(g.resume && 2 * n <= (unsigned)g.few))
+        // few blocks: eight wavefronts halve a rank step's latency
+        if (nw == 4 && 2 * n > (unsigned)g.few)
             aca_wide_kernel<KIND, DIM, TOL, 4><<<m, 4 * kWave, 0, s>>>(g);
         else
             aca_wide_kernel<KIND, DIM, TOL, 8><<<m, 8 * kWave, 0, s>>>(g);

@@ -712,9 +712,9 @@ constexpr int kRegTries = 64, kWideTries = 32, kWideRetries = 8;
 // cost most, where such blocks make rounds in any case (N = 16384, 2D uniform 15.5 and 17.4).
 constexpr int64_t kSearchAlone = (int64_t)1 << 22;
 constexpr int kAcaBlind = 4;  // rounds between two looks at the queues
-// Bounds of a wide class' slabs together: of an engine with two streams, and of one with a
-// single stream, which shares the chip with other such engines
-constexpr int64_t kSlabBytes = (int64_t)3 << 30, kSlabShared = (int64_t)256 << 20;
+// Bound of a wide class' slabs together of an engine with one stream, which shares the chip
+// with other such engines (otherwise: Engine::aca_slab_bytes)
+constexpr int64_t kSlabShared = (int64_t)256 << 20;
 
 static int aca_class(const Engine& eng, const KernelParams& kp, int a)
 {
@@ -824,6 +824,7 @@ struct AcaWork {
     DevBuf<int> own_ints;
     DevBuf<double> own_fro2, own_slabs[kWide];
     hipStream_t s = nullptr, s2 = nullptr;
+    int64_t bound = 0;  // of a wide class' slabs
     bool running = false;
     ~AcaWork()
     {
@@ -845,6 +846,7 @@ struct AcaWork {
     {
         s = eng.stream;
         s2 = eng.stream2;
+        bound = eng.aca_slab_bytes;
         int dev = 0;
         HMG_HIP(hipGetDevice(&dev));
         HMG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -856,8 +858,8 @@ struct AcaWork {
     int slab_count(const AcaCounts& cnt, int i) const
     {
         const int n = cnt.n[kRegClass + i];
-        if (n == 0) return 0;
-        const int64_t fit = (shared() ? kSlabShared : kSlabBytes) / (std::max<int64_t>(cnt.slab[i], 1) * 8);
+        if (n == 0 || bound == 0) return 0;
+        const int64_t fit = (shared() ? std::min(kSlabShared, bound) : bound) / (std::max<int64_t>(cnt.slab[i], 1) * 8);
         return (int)std::min<int64_t>(std::min(n, std::max(cus, 1) * (i == 0 ? 1 : 3)), std::max<int64_t>(fit, 1));
     }
 };

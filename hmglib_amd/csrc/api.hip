@@ -1634,6 +1634,13 @@ hmg_status hmg_set_option(struct h_matrix_data* data, int option, int64_t value)
         }
         e->aca_lds_pad = (int)value;
         return HMG_OK;
+    case HMG_OPT_ACA_SLAB_BYTES:
+        if (value < 0) {
+            set_error("ACA slab bytes must not be negative");
+            return HMG_ERR_INVALID;
+        }
+        e->aca_slab_bytes = value;
+        return HMG_OK;
     case HMG_OPT_MIXED_ACA_PARTS:
         if (value < 1 || value > 4096) {
             set_error("mixed ACA parts must be in 1..4096");

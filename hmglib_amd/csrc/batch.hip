@@ -119,6 +119,7 @@ hmg_status run_group(h_matrix_data* const* data, const std::vector<int>& members
     v.nblocks = (int)na;
     v.aca_row_scan = e0->aca_row_scan;
     v.aca_big_entries = e0->aca_big_entries;
+    v.aca_slab_bytes = e0->aca_slab_bytes;
     v.aca_huge_entries = e0->aca_huge_entries;
     v.aca_tol_mode = e0->aca_tol_mode;
     v.aca_tol_c = e0->aca_tol_c;

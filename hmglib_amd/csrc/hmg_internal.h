@@ -484,6 +484,7 @@ struct Engine {
     // from h_fly_sym on the symmetric ones); chunk size of the work items (0: none yet)
     std::vector<int> h_fly_ptr, h_fly_sym, h_fly_blk;
     int near_scale = 0;
+    int64_t aca_slab_bytes = (int64_t)3 << 30;  // bound of a wide class' slabs (0: none)
     int64_t lr_elems = 0;  // elements of the factors at the layout's ranks
     int layout_k = -1;  // rank bound of the present layout (aca_layout), -1: none
     // matrix-free near field (symmetric when both sets are the same points)

@@ -280,7 +280,12 @@ hmg_status hmg_get_schedule(const struct h_matrix_data* data, int64_t out[11]);
  *   factors' size (at least 1 GiB); results unchanged.
  * HMG_OPT_ACA_LDS_BYTES [0]: unused LDS each workgroup of the main launch of the
  *   same blocks reserves, capping the blocks in flight per compute unit (their factor columns,
- *   re-read at every rank step, then stay in cache); results unchanged. */
+ *   re-read at every rank step, then stay in cache); results unchanged.
+ * HMG_OPT_ACA_SLAB_BYTES [3221225472]: bound of the scratch in which the wide blocks
+ *   of the ACA (more than 1024 rows or columns, other than those kept in memory)
+ *   hold V, per class of blocks (at least one block at a time).  0, or where not
+ *   even that is free: those blocks keep their factors in memory, on 8 wavefronts
+ *   each (same factors up to the rounding of the norms). */
 #define HMG_OPT_NEAR_SYMMETRIC 1
 #define HMG_OPT_NEAR_LDS_BYTES 2
 #define HMG_OPT_SERIALIZE 3
@@ -296,6 +301,7 @@ hmg_status hmg_get_schedule(const struct h_matrix_data* data, int64_t out[11]);
 #define HMG_OPT_LR_PRIORITY 13
 #define HMG_OPT_MIXED_ACA_PARTS 14
 #define HMG_OPT_ACA_LDS_BYTES 15
+#define HMG_OPT_ACA_SLAB_BYTES 16
 #define HMG_PREC_FP64 0
 #define HMG_PREC_MIXED 1
 hmg_status hmg_set_option(struct h_matrix_data* data, int option, int64_t value);

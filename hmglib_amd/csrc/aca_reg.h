@@ -72,13 +72,14 @@ struct AcaArgs {
 };
 
 constexpr int kRegSlots = 1;    // rows and columns per thread
+static_assert(kRegSlots == 1, "the look-ahead over rejected rows takes the first slot only");
 constexpr int kRegTail = 8;     // rank terms in LDS after the ones in registers
 constexpr int kRegRank = 64;    // largest rank of the register form
 // rows of one workgroup of the search over suspended blocks
 constexpr int kSearchRows = kWave;
 
-// Launches the g.nlist blocks of g.list[] on teams of nw wavefronts: 1, 2, 3, 5, 9 or 12
-// (every block within 64 nw rows and columns), or with wide set 4 or 8 (blocks of any
+// Launches the g.nlist blocks of g.list[] on teams of nw wavefronts: 1, 2, 3, 4, 5, 8, 9, 12
+// or 16 (every block within 64 nw rows and columns), or with wide set 4 or 8 (blocks of any
 // size; a slab holds at least k x m2 elements of each).  Dimension 2 or 3; kmax: the
 // largest rank among the blocks.  One translation unit per kernel kind.
 template <int KIND>

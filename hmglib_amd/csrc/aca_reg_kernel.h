@@ -327,7 +327,8 @@ __device__ __forceinline__ void reg_publish(double* s, const RegRow<NT> (&f)[kRe
 // cache.  Of N = 262144 points in 3D, leaf 256, k = 24 (exponential): blocks up to 512 take
 // 0.25 us each on 8 wavefronts (two teams per compute unit) against 0.42 on 9 (one), up
 // to 320 0.21 on 5 with NT = 8 against 0.28 with 16, up to 256 0.11 on 4.  The whole build
-// runs 54 ms of these kernels; the memory form took 150.  No variant uses scratch.
+// runs 54 ms of these kernels; the memory form took 150.  No variant of this kernel uses
+// scratch memory.
 template <int KIND, int DIM, bool TOL, int NW, int NT>
 __global__ void __launch_bounds__(NW* kWave) __attribute__((amdgpu_waves_per_eu(reg_waves(NT), reg_waves(NT))))
 aca_reg_kernel(AcaArgs g)
@@ -729,7 +730,8 @@ aca_reg_kernel(AcaArgs g)
 // that every factor read is a run of consecutive values, four columns (rows) per
 // thread at a time with eight terms of each in flight.  The slab is written to V_b at the end.
 // Bound by those reads (ranks^2 / 2 terms per row, past the L2 for many blocks at once):
-// about 9 TB/s at N = 262144 in 3D, 22 ms of that build.
+// about 9 TB/s at N = 262144 in 3D, 22 ms of that build.  At three wavefronts per SIMD (168
+// registers) the variants spill 4 to 12 of them (20 to 52 bytes a lane of scratch memory).
 // Sums over columns or rows are formed as a team of kWideWaves wavefronts forms them (one
 // partial sum per thread of such a team, reduced per wavefront, added in order), whatever
 // NW: a smaller team holds several of its threads' sums.  A block's ranks and factors then

@@ -72,10 +72,13 @@ __device__ __forceinline__ double exp_nonpos(double x)
     return ldexp(p, __double2loint(m));
 }
 
-// sqrt(x) for finite x >= 0: the hardware reciprocal square root (22 bits; its infinity
-// at 0 made finite), a Goldschmidt step (44 bits) and one Newton correction of the root,
-// g += (x - g^2) h, whose error is its final rounding.  Correctly rounded in 5 10^6
-// random arguments, as with a refined h and a second correction.
+// sqrt(x) for finite x >= 0: the hardware reciprocal square root (relative error at most
+// 2^-24.2 in 8.4 10^9 random arguments on MI355X; its infinity at 0 made finite), a
+// Goldschmidt step and one Newton correction of the root, g += (x - g^2) h with the
+// unrefined h, whose error is its final rounding but for 2^-13 ulp or so: 214 of those
+// arguments were rounded to the other neighbour, none with a refined h or a second
+// correction.  (An entry's error is that of the exponential: at most 0.86 ulp in all, 0.89
+// with the exact root and the longer exponential.)
 __device__ __forceinline__ double sqrt_nonneg(double x)
 {
     const double y = fmin(__builtin_amdgcn_rsq(x), 1.0e300);

@@ -713,8 +713,10 @@ constexpr int kRegTries = 64, kWideTries = 32, kWideRetries = 8;
 constexpr int64_t kSearchAlone = (int64_t)1 << 22;
 constexpr int kAcaBlind = 4;  // rounds between two looks at the queues
 // Bound of a wide class' slabs together of an engine with one stream, which shares the chip
-// with other such engines (otherwise: Engine::aca_slab_bytes)
-constexpr int64_t kSlabShared = (int64_t)256 << 20;
+// with other such engines and keeps it (otherwise: Engine::aca_slab_bytes).  With 256 MB the
+// longest builds of a server (N = 262144, one of three slots) took 12 % longer, with 3 GiB
+// eight slots would keep 48.
+constexpr int64_t kSlabShared = (int64_t)1 << 30;
 
 static int aca_class(const Engine& eng, const KernelParams& kp, int a)
 {

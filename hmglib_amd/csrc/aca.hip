@@ -742,6 +742,7 @@ struct AcaCounts {
     int kmax[kClasses] = {0};
     int m1max[kClasses] = {0};
     int64_t area[kClasses] = {0};   // largest block's entries
+    double work[kClasses] = {0.0};  // rows and columns times rank
     int64_t slab[kWide] = {0};
 };
 
@@ -774,6 +775,7 @@ static AcaCounts aca_order(const Engine& eng, const KernelParams& kp, const std:
         const int a = members[q], i = cls[q];
         const int4 b = eng.h_blk[eng.ndense + a];
         c.m1max[i] = std::max(c.m1max[i], b.y - b.x + 1);
+        c.work[i] += ((double)(b.y - b.x + 1) + (b.w - b.z + 1)) * eng.h_kb[a];
         c.area[i] = std::max(c.area[i], (int64_t)(b.y - b.x + 1) * (b.w - b.z + 1));
         if (i >= kRegClass && i < kRegClass + kWide)
             c.slab[i - kRegClass] = std::max(c.slab[i - kRegClass], (int64_t)(b.w - b.z + 1) * eng.h_kb[a]);
@@ -881,8 +883,8 @@ int64_t aca_work_bytes(const Engine& eng, const KernelParams& kp)
 // About how long n teams of class c run (us): a rank step's latency by team and block size
 // (a team of 16 wavefronts 24 us, of one 6; a wide one 50 at 4096 columns), the ranks, and
 // the teams that a compute unit runs one after another.  Dealt by rows, columns and ranks
-// alone, small builds left one stream idle for a third of the time (N = 4096, 2D clouds, ACA
-// 3.2 ms).
+// alone, small builds left one stream idle for a third of the time (ACA of N = 4096, 2D
+// uniform 1.62 ms so, 1.72 that way).
 static double class_time(const AcaCounts& cnt, int c, int n, int cus)
 {
     const int nw = kRegWaves[c - kRegClass];
@@ -893,8 +895,8 @@ static double class_time(const AcaCounts& cnt, int c, int n, int cus)
 
 // The blocks of list[] (aca_order), factor offsets uoff / voff (leading dims eng.ldu /
 // eng.ldv) into U / V or block pointers ublk / vblk.  The classes are dealt to the
-// engine's two streams, the longest first, to the one with less to do so far, so that one's
-// last workgroups run beside the next; both are joined back.  Rounds: blocks that suspended themselves are searched and resumed until
+// engine's two streams, each to the one with less to do so far, so that one's last
+// workgroups run beside the next; both are joined back.  Rounds: blocks that suspended themselves are searched and resumed until
 // none is left (each round raises the rank or the row of every one of them); the host
 // looks at the queues once per kAcaBlind rounds, the launches in between end at once
 // where their queue is empty.
@@ -1008,16 +1010,23 @@ static hmg_status aca_launch(Engine& eng, const Coords& c1, const Coords& c2, co
         HMG_HIP(hipGetLastError());
         n[c] = 0;
     }
+    // Does the build fill the chip several times over?  Its classes' work counts then, and the
+    // wide ones go first (3D, N = 262144: 60.5 ms; longest first 63.1)
+    double teams = 0.0;
     bool rounds_anyway = false;
-    for (int c = kRegClass; c < kClasses; c++) rounds_anyway = rounds_anyway || cnt.area[c] > kSearchAlone;
+    for (int c = kRegClass; c < kClasses; c++) {
+        teams += (double)cnt.n[c] * kRegWaves[c - kRegClass] / (12.0 * std::max(work.cus, 1));
+        rounds_anyway = rounds_anyway || cnt.area[c] > kSearchAlone;
+    }
+    const bool filled = teams > 8.0;
     for (int round = 0; nreg > 0;) {
         // one look: the blocks themselves, or kAcaBlind rounds of the suspended ones
         const int rounds = round == 0 ? 1 : kAcaBlind;
         double load[2] = {0.0, 0.0};
         std::vector<std::pair<double, int>> deal;
         for (int c = kRegClass; c < kClasses; c++)
-            if (n[c] > 0) deal.emplace_back(class_time(cnt, c, n[c], work.cus), c);
-        std::sort(deal.begin(), deal.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+            if (n[c] > 0) deal.emplace_back(filled ? cnt.work[c] * n[c] / cnt.n[c] : class_time(cnt, c, n[c], work.cus), c);
+        if (!filled) std::sort(deal.begin(), deal.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
         for (const auto& [time, c] : deal) {
             const bool wide = c < kRegClass + kWide;
             const int to = load[0] <= load[1] ? 0 : 1;

@@ -1,4 +1,4 @@
-// mvp.hip -- H-matrix-vector products, near-field fill, dense checker products.
+// mvp.hip -- H-matrix-vector products, near-field fill, dense products of the tests.
 //
 // y = P1^T ( sum_dense A_b x~_J + sum_aca U_b (V_b^T x~_J) ),  x~ = P2 x
 // (reference: hmglib.cu:271-286, linear_algebra.cu:4292-4379, 1429-1591,
@@ -556,7 +556,7 @@ void launch_full(unsigned grid, hipStream_t s, const Coords& c1, const Coords& c
         full_kernel<KIND, 0><<<grid, kThreads, 0, s>>>(c1, c2, kp, xs, chunk, nchunks, nitems, P, ld);
 }
 
-// exact rows (checker at scale): one wavefront per sampled row
+// exact rows (the reference at scale): one wavefront per sampled row
 __global__ void __launch_bounds__(kThreads)
 rows_kernel(Coords c1, Coords c2, KernelParams kp, const double* __restrict__ xs,
             const int64_t* __restrict__ rows, const int64_t* __restrict__ inv1, int nrows,

@@ -190,7 +190,7 @@ hmg_status hmg_apply_h_matrix_mvp_noalloc(const double* X, double* Y, int nrhs, 
  * workgroup form).  Needs precompute_aca. */
 hmg_status hmg_autotune_product(struct h_matrix_data* data, const double* X, double* Y, int nrhs, int reps,
                                 int64_t out[4]);
-/* dense product for nrhs right-hand sides on sampled ORIGINAL rows (checker helper
+/* dense product for nrhs right-hand sides on sampled ORIGINAL rows (reference helper
  * at scale): Yrows[q + c*nrows] = sum_j K(rows[q], j) X[j + c*n2]. rows is a device
  * int64 array. */
 hmg_status hmg_dense_rows(const double* X, int nrhs, const int64_t* rows, int nrows, double* Yrows,

@@ -1,6 +1,6 @@
 """ctypes front-end of the CPU oracle (oracle/libhmg_oracle.so).
 
-TEST INFRASTRUCTURE ONLY: the checker for the HIP engine.  Imported only by
+TEST INFRASTRUCTURE ONLY: the oracle for the HIP engine.  Imported only by
 tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg -- never by the
 product package hmglib_amd.
 """

@@ -1,7 +1,7 @@
 /*
  * hmg_oracle.c -- CPU restatement of hmglib's H-matrix build + H-MVP path.
  *
- * TEST INFRASTRUCTURE ONLY (the checker).  See hmg_oracle.h for what pins each
+ * TEST INFRASTRUCTURE ONLY (the oracle).  See hmg_oracle.h for what pins each
  * function.  Reference citations are file:line in hmglib's src/ directory.
  *
  * Build: gcc -O2 -fopenmp -ffp-contract=off -fPIC -shared (oracle/Makefile).

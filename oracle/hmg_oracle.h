@@ -1,7 +1,7 @@
 /*
  * hmg_oracle.h -- CPU restatement of hmglib's H-matrix build + H-MVP path.
  *
- * TEST INFRASTRUCTURE ONLY.  This library is the checker: only tests/,
+ * TEST INFRASTRUCTURE ONLY.  This library is the oracle: only tests/,
  * __graft_entry__.smoke() and bench.py's cpu_baseline leg may load it.  The
  * product (hmglib_amd/libhmglib.so) never links, calls or falls back to it.
  *
